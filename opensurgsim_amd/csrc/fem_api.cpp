@@ -15,6 +15,7 @@
 #include "fem_hex.hpp"
 #include "fem_lu.hpp"
 #include "fem_mcg.hpp"
+#include "fem_resident.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -25,6 +26,7 @@
 #include <cstring>
 #include <limits>
 #include <map>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -238,6 +240,16 @@ struct fem_ctx {
     DevBuf<unsigned char> cg_x2;  // FP32 refinement: inner solution of the odd sweeps
     DevBuf<unsigned char> cg_r1, cg_z1, cg_q1, cg_w0, cg_w1;                    // fused CG: second buffers
     DevBuf<double> part7;      // [2][kFusedSums * kCgBlocks] block sums of the fused CG kernel, by parity
+    // one-launch CG solves (fem_resident.hip): the partition for res_precision, exchanged vectors, published sums
+    ResidentTables res;
+    int res_precision = -1;
+    std::vector<double> h_x0;  // rest positions, for the partition
+    bool res_dirty = false;    // the exchanged vectors have to be emptied (new, or left by a solve that gave up)
+    int res_backoff = 0;       // solves left to run with one launch per iteration after one gave up
+    DevBuf<unsigned char> res_mem, res_exch;
+    DevBuf<unsigned long long> res_slots;
+    int num_cus = 0;
+    long long res_wait_ticks = 400000;  // 4 ms; FEM_CG_WAIT_US
     DevBuf<double> partial;    // [4 * kCgBlocks] block sums of the grid reductions
     DevBuf<CgScalars> scal;    // [0] inner/FP64 solve, [1] outer refinement
     DevBuf<CgScalars> time_sc; // operator replay timing (fem_time_operator)
@@ -477,6 +489,83 @@ Operator op_of(fem_ctx* c) {
     return o;
 }
 
+// The partition of a one-launch solve in this precision, built on its first use for the mesh; none (groups == 0)
+// when the operator does not fit the chip.
+void ensure_resident(fem_ctx* c, bool fp32) {
+    if (c->res_precision == (fp32 ? 1 : 0)) return;
+    c->res = ResidentTables{};
+    c->res_precision = fp32 ? 1 : 0;
+    if (c->cg_kernels != 0 || c->kind == FEM_ELEMENT_HEX || c->num_instances > 0) return;
+    const ResidentPlan plan = plan_resident(c->num_nodes, c->h_rowptr_b.data(), c->h_colidx_b.data(), c->h_x0.data(),
+                                            fp32, c->num_cus);
+    if (plan.groups == 0) return;
+    std::vector<unsigned char> h;
+    std::vector<size_t> at;
+    auto add = [&](const auto& v) {
+        at.push_back(h.size());
+        const auto* p = reinterpret_cast<const unsigned char*>(v.data());
+        h.insert(h.end(), p, p + v.size() * sizeof(v[0]));
+        h.resize((h.size() + 255) & ~size_t(255));
+    };
+    add(plan.group);
+    add(plan.row_node);
+    add(plan.halo_node);
+    add(plan.halo_pos);
+    add(plan.lane_k0);
+    add(plan.lane_info);
+    add(plan.row_lane);
+    add(plan.cols);
+    c->res_mem.alloc(h.size());
+    c->res_mem.upload(h.data(), h.size(), c->stream);
+    c->res_exch.alloc(2 * (size_t)c->num_nodes * (fp32 ? kResRowBytes32 : kResRowBytes64));
+    c->res_dirty = true;
+    if (!c->res_slots.p) c->res_slots.alloc(kResSlotWords);
+    HIPCHECK(hipStreamSynchronize(c->stream));
+    unsigned char* p = c->res_mem.p;
+    c->res.nb = plan.nb;
+    c->res.max_cols = plan.max_cols;
+    c->res.group = reinterpret_cast<const int4*>(p + at[0]);
+    c->res.row_node = reinterpret_cast<const int*>(p + at[1]);
+    c->res.halo_node = reinterpret_cast<const int*>(p + at[2]);
+    c->res.halo_pos = reinterpret_cast<const int*>(p + at[3]);
+    c->res.lane_k0 = reinterpret_cast<const int*>(p + at[4]);
+    c->res.lane_info = reinterpret_cast<const int*>(p + at[5]);
+    c->res.row_lane = reinterpret_cast<const uint16_t*>(p + at[6]);
+    c->res.cols = reinterpret_cast<const uint16_t*>(p + at[7]);
+    c->res.groups = plan.groups;
+}
+
+bool use_resident(const fem_ctx* c, bool fp32) {
+    return c->res.groups > 0 && c->res_precision == (fp32 ? 1 : 0) && c->res_backoff == 0;
+}
+
+// One-launch solves of a device go one after another: two of them side by side could each hold CUs that the other's
+// workgroups wait for. Held from the launch until the host has seen the solve's end.
+std::mutex& resident_mutex(int device) {
+    static std::mutex mu[64];
+    return mu[(unsigned)device % 64];
+}
+
+void launch_resident(fem_ctx* c, const CgArgs& a, int max_iter) {
+    if (c->res_dirty) {
+        HIPCHECK(hipMemsetAsync(c->res_exch.p, 0, c->res_exch.n, c->stream));
+        c->res_dirty = false;
+    }
+    ResidentArgs r;
+    r.t = c->res;
+    r.S = a.S;
+    r.r = a.r1;
+    r.z = a.z1;
+    r.x = a.x;
+    r.dinv = a.fp32 ? a.binv : a.dinv;
+    r.exch = c->res_exch.p;
+    r.slots = c->res_slots.p;
+    r.sc = a.sc;
+    r.max_iter = max_iter;
+    r.wait_ticks = c->res_wait_ticks;
+    launch_cg_resident(r, a.fp32, c->stream);
+}
+
 CgArgs cg_args(fem_ctx* c, bool fp32, double tol) {
     CgArgs a;
     a.op = op_of(c);
@@ -500,6 +589,7 @@ CgArgs cg_args(fem_ctx* c, bool fp32, double tol) {
     a.w[1] = c->cg_w1.p;
     a.part7 = c->part7.p;
     a.binv = c->cg_binv.p;
+    a.slots = use_resident(c, fp32) ? c->res_slots.p : nullptr;
     return a;
 }
 
@@ -542,10 +632,30 @@ int64_t max_iters(fem_ctx* c) {
     return std::min<int64_t>(m, std::numeric_limits<int>::max() - 1);
 }
 
-// Runs the CG iterations of an initialised solve: launches a predicted number of iterations, then
-// polls the device 'done' flag between chunks. Returns the iteration count.
-int run_cg_iterations(fem_ctx* c, const CgArgs& a, int max_iter) {
+constexpr int kResBackoff = 256;  // solves with one launch per iteration after a one-launch solve gave up
+
+// Runs the CG iterations of an initialised solve of right-hand side b: in one launch where the operator fits the
+// chip (a.slots), otherwise launches a predicted number of iterations, then polls the device 'done' flag between
+// chunks. Returns the iteration count.
+int run_cg_iterations(fem_ctx* c, const CgArgs& a, const double* b, int max_iter) {
     int& pred = c->solving_adjoint ? c->predicted_adj : c->predicted_iters;
+    if (a.slots) {
+        std::lock_guard<std::mutex> one(resident_mutex(c->device));
+        TIMED(c, FEM_PHASE_SPMV, 0, launch_resident(c, a, max_iter));
+        HIPCHECK(hipMemcpyAsync(c->h_sc, a.sc, sizeof(CgScalars), hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(hipStreamSynchronize(c->stream));
+        if (c->timer.enabled) c->timer.resolve();
+        if (!c->h_sc->pad) {
+            pred = c->h_sc->iters + 1;
+            return c->h_sc->iters;
+        }
+        // gave up waiting for a workgroup: started over with one launch per iteration, as are the next solves
+        c->res_backoff = kResBackoff;
+        c->res_dirty = true;
+        CgArgs t = a;
+        t.slots = nullptr;
+        launch_solver_init(c, t, b, nullptr);
+    }
     int k = 0;
     // iteration k = convergence test of k-1 + p update + operator application, then vector updates;
     // the last launch (k == max_iter) only tests.
@@ -620,11 +730,14 @@ void linear_solve(fem_ctx* c) {
     const bool fp32 = c->opt.precision == FEM_PRECISION_FP32_REFINED;
     const int max_iter = (int)max_iters(c);
     size_t n = (size_t)c->ndof;
+    ensure_resident(c, fp32);
+    if (c->res_backoff > 0) --c->res_backoff;
     if (!fp32) {
         CgArgs a = cg_args(c, false, c->opt.cg_tolerance);
+        if (max_iter < 1) a.slots = nullptr;
         a.x = c->dv.p;
         TIMED(c, FEM_PHASE_CG_INIT, 0, launch_solver_init(c, a, c->b.p, nullptr));
-        int it = run_cg_iterations(c, a, max_iter);
+        int it = run_cg_iterations(c, a, c->b.p, max_iter);
         c->stats.last_cg_iterations = it;
         c->stats.total_cg_iterations += it;
         c->stats.last_cg_error = c->h_sc->err;
@@ -648,6 +761,9 @@ void linear_solve(fem_ctx* c) {
     }
     CgArgs a = cg_args(c, true, c->opt.inner_tolerance);
     a.floor_tol = kInnerFloor * c->opt.cg_tolerance;
+    if (max_iter < 1) a.slots = nullptr;
+    std::unique_lock<std::mutex> one(resident_mutex(c->device), std::defer_lock);
+    if (a.slots) one.lock();
     CgScalars* outer = c->scal.p + 1;
     // One-kernel CG path: sweep s is one launch for dv_s = dv_{s-1} + x_{s-1}, the FP64 residual and the inner
     // solve's start, and one for the outer test with the inner scalars; dv_s and x_s alternate between two
@@ -666,7 +782,7 @@ void linear_solve(fem_ctx* c) {
                                       dvb[sweep & 1], sweep == 0, xb[sweep & 1], (float*)a.r1, (float*)a.z1,
                                       (float*)a.binv, c->partial.p, outer, c->stream));
             launch_refine_check_init(c->partial.p, sweep, c->opt.cg_tolerance, c->opt.inner_tolerance, outer, a.sc,
-                                     c->refine_iters.p, max_ref + 1, c->stream);
+                                     c->refine_iters.p, max_ref + 1, a.slots, c->stream);
             return;
         }
         TIMED(c, FEM_PHASE_REFINE, 0,
@@ -683,6 +799,10 @@ void linear_solve(fem_ctx* c) {
         if (fused) {
             CgArgs ai = a;
             ai.x = xb[sweep & 1];
+            if (a.slots) {
+                TIMED(c, FEM_PHASE_SPMV, sweep << 20, launch_resident(c, ai, cap));
+                return;
+            }
             for (int k = 0; k <= cap; ++k) launch_iteration(c, ai, k, cap, (sweep << 20) | k);
             return;
         }
@@ -711,6 +831,13 @@ void linear_solve(fem_ctx* c) {
         ++sweep;
         check(sweep);
         read_back(sweep);
+    }
+    if (a.slots && c->h_sc[1].pad) {
+        // an inner solve gave up waiting for a workgroup: the solve starts over with one launch per iteration
+        c->res_backoff = kResBackoff;
+        c->res_dirty = true;
+        one.unlock();
+        return linear_solve(c);
     }
     // sweeps that applied a correction recorded their inner iteration counts
     int total = 0, sweeps = 0;
@@ -1936,6 +2063,7 @@ int fem_create(int device, fem_ctx** out) {
         HIPCHECK(hipSetDevice(device));
         HIPCHECK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
         c->own_stream = true;
+        HIPCHECK(hipDeviceGetAttribute(&c->num_cus, hipDeviceAttributeMultiprocessorCount, device));
         c->scratch = noalloc_scratch_address(device);  // once per device, with the device current
         HIPCHECK(hipHostMalloc((void**)&c->h_sc, 2 * sizeof(CgScalars), hipHostMallocDefault));
         HIPCHECK(hipHostMalloc((void**)&c->h_counters, 8 * sizeof(int), hipHostMallocDefault));
@@ -1950,6 +2078,7 @@ int fem_create(int device, fem_ctx** out) {
         for (int i = 0; i < 16; ++i) c->predicted_sweep[i] = 32;
         if (const char* e = std::getenv("FEM_CG_KERNELS"))
             c->cg_kernels = std::strcmp(e, "fused") == 0 ? 1 : std::strcmp(e, "split") == 0 ? 2 : 0;
+        if (const char* e = std::getenv("FEM_CG_WAIT_US")) c->res_wait_ticks = 100 * std::max(0ll, std::atoll(e));
         for (int i = 0; i < 17; ++i) c->predicted_hex[i] = 8;
         std::memset(&c->stats, 0, sizeof(c->stats));
         c->stats.active = 1;
@@ -2078,6 +2207,7 @@ int fem_upload_mesh(fem_ctx* c, int kind, int64_t num_nodes, const double* x0, i
                 HIPCHECK(hipStreamSynchronize(c->stream));  // the host tables are freed on return
             }
             build_tet_maps(c, conn);
+            c->h_x0.assign(x0, x0 + 3 * num_nodes);
             std::vector<int4> c4(num_elements);
             for (int64_t e = 0; e < num_elements; ++e)
                 c4[e] = make_int4(conn[4 * e], conn[4 * e + 1], conn[4 * e + 2], conn[4 * e + 3]);
@@ -2175,6 +2305,8 @@ int fem_set_options(fem_ctx* c, const fem_options* o) {
         if (c->mesh_ready) {
             HIPCHECK(hipSetDevice(c->device));
             alloc_precision_buffers(c);
+            if (c->opt.linear_solver == FEM_LINEAR_SOLVER_CG)
+                ensure_resident(c, c->opt.precision == FEM_PRECISION_FP32_REFINED);
         }
         return FEM_OK;
     });

@@ -13,6 +13,7 @@
 #include "fem_device.hpp"
 #include "fem_kernels.hpp"
 #include "fem_reduce.hpp"
+#include "fem_resident.hpp"
 
 #include <algorithm>
 #include <cfloat>
@@ -584,12 +585,20 @@ __global__ __launch_bounds__(kCgThreads) void cg_init_guess_kernel(Operator op, 
     if (threadIdx.x == 0) partial[2 * kCgBlocks + blockIdx.x] = srr;
 }
 
+// The published sums of a one-launch solve that follows, emptied (one workgroup).
+__device__ __forceinline__ void empty_slots(unsigned long long* slots) {
+    if (slots)
+        for (size_t i = threadIdx.x; i < kResSlotWords; i += blockDim.x) slots[i] = kResEmpty;
+}
+
 // Scalars of a solve started from a guess: threshold max(tol^2 |b|^2, realmin); Eigen's exit before the first
 // iteration when |r|^2 is already below it (err = |r| / |b|), or when b = 0 (x = 0).
 __global__ __launch_bounds__(kCgThreads) void cg_init2_guess_kernel(const double* __restrict__ partial, CgScalars* sc,
-                                                                    double tol, double* __restrict__ x, int n) {
+                                                                    double tol, double* __restrict__ x, int n,
+                                                                    unsigned long long* __restrict__ slots) {
     __shared__ double lds[64];
     __shared__ int exit_zero;
+    empty_slots(slots);
     double bb, rz, rr;
     reduce_partials3(partial, partial + kCgBlocks, partial + 2 * kCgBlocks, bb, rz, rr, lds);
     if (threadIdx.x == 0) {
@@ -601,6 +610,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_init2_guess_kernel(const double
         sc->iters = 0;
         sc->err = 0.0;
         sc->converged = 0;
+        sc->pad = 0;
         sc->done = 0;
         exit_zero = 0;
         if (bb == 0.0) {
@@ -623,9 +633,11 @@ __global__ __launch_bounds__(kCgThreads) void cg_init2_guess_kernel(const double
 // its solution only has to bring the outer residual below the outer tolerance.
 __global__ __launch_bounds__(kCgThreads) void cg_init2_kernel(const double* __restrict__ partial, CgScalars* sc,
                                                               const CgScalars* __restrict__ skip, double tol,
-                                                              double floor_tol) {
+                                                              double floor_tol,
+                                                              unsigned long long* __restrict__ slots) {
     __shared__ double lds[64];
     if (skip && skip->done) return;
+    empty_slots(slots);
     double bb, rz;
     reduce_partials2(partial, partial + kCgBlocks, bb, rz, lds);
     if (threadIdx.x == 0) {
@@ -639,6 +651,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_init2_kernel(const double* __re
         sc->iters = 0;
         sc->err = 0.0;
         sc->converged = 0;
+        sc->pad = 0;
         sc->done = 0;
         if (bb == 0.0) {
             sc->done = 1;
@@ -1071,19 +1084,22 @@ void launch_cg_init(const CgArgs& a, const double* b, const CgScalars* skip, hip
     else
         launch_k((cg_init_kernel<double>), grid, block, 0, s, a.op, (const double*)a.S, b, (double*)a.x,
                            (double*)a.r, (double*)a.z, (double*)a.dinv, a.partial, skip);
-    launch_k(cg_init2_kernel, dim3(1), block, 0, s, a.partial, a.sc, skip, a.tol, a.floor_tol);
+    launch_k(cg_init2_kernel, dim3(1), block, 0, s, a.partial, a.sc, skip, a.tol, a.floor_tol,
+             a.slots);
 }
 
 void launch_cg_init_guess(const CgArgs& a, const double* b, hipStream_t s) {
     launch_k(cg_init_guess_kernel, dim3(kCgBlocks), dim3(kCgThreads), 0, s, a.op, (const double*)a.S, b,
              (const double*)a.x, (double*)a.r, (double*)a.z, (double*)a.dinv, a.partial);
-    launch_k(cg_init2_guess_kernel, dim3(1), dim3(kCgThreads), 0, s, a.partial, a.sc, a.tol, (double*)a.x, a.n);
+    launch_k(cg_init2_guess_kernel, dim3(1), dim3(kCgThreads), 0, s, a.partial, a.sc, a.tol, (double*)a.x, a.n,
+             a.slots);
 }
 
 void launch_cg_init_block(const CgArgs& a, const double* b, const CgScalars* skip, hipStream_t s) {
     launch_k(cg_init_block_kernel, dim3(kCgBlocks), dim3(kCgThreads), 0, s, a.op, (const float*)a.S, b, (float*)a.x,
              (float*)a.r, (float*)a.z, (float*)a.binv, a.partial, skip);
-    launch_k(cg_init2_kernel, dim3(1), dim3(kCgThreads), 0, s, a.partial, a.sc, skip, a.tol, a.floor_tol);
+    launch_k(cg_init2_kernel, dim3(1), dim3(kCgThreads), 0, s, a.partial, a.sc, skip, a.tol, a.floor_tol,
+             a.slots);
 }
 
 void launch_cg_apply(const CgArgs& a, int k, int max_iter, hipStream_t s) {
@@ -1100,7 +1116,8 @@ void launch_cg_apply(const CgArgs& a, int k, int max_iter, hipStream_t s) {
 
 void launch_cg_init2(const double* partial, CgScalars* sc, const CgScalars* skip, double tol, hipStream_t s,
                      double floor_tol) {
-    launch_k(cg_init2_kernel, dim3(1), dim3(kCgThreads), 0, s, partial, sc, skip, tol, floor_tol);
+    launch_k(cg_init2_kernel, dim3(1), dim3(kCgThreads), 0, s, partial, sc, skip, tol, floor_tol,
+             (unsigned long long*)nullptr);
 }
 
 void launch_cg_vector_raw(bool fp32, int n, int k, void* x, void* r, void* z, const void* p, const void* q,
@@ -1320,9 +1337,11 @@ __global__ __launch_bounds__(kCgThreads) void refine_sweep_kernel(
 __global__ __launch_bounds__(kCgThreads) void refine_check_init_kernel(const double* __restrict__ partial, int sweep,
                                                                        double tol, double inner_tol,
                                                                        CgScalars* outer, CgScalars* inner,
-                                                                       int* __restrict__ refine_iters, int nrec) {
+                                                                       int* __restrict__ refine_iters, int nrec,
+                                                                       unsigned long long* __restrict__ slots) {
     __shared__ double lds[64];
     if (sweep > 0 && outer->done) return;
+    empty_slots(slots);
     double rr, bb, rz;
     reduce_partials3(partial + 3 * kCgBlocks, partial, partial + kCgBlocks, rr, bb, rz, lds);
     if (threadIdx.x == 0) {
@@ -1333,8 +1352,10 @@ __global__ __launch_bounds__(kCgThreads) void refine_check_init_kernel(const dou
             outer->iters = 0;
             outer->done = 0;
             outer->converged = 0;
+            outer->pad = 0;
         } else {
             refine_iters[sweep - 1] = inner->iters;
+            if (inner->pad) outer->pad = 1;  // the solve starts over (the host reads the outer scalars)
         }
         outer->rr = rr;
         outer->err = outer->bb > 0 ? sqrt(rr / outer->bb) : 0.0;
@@ -1353,6 +1374,7 @@ __global__ __launch_bounds__(kCgThreads) void refine_check_init_kernel(const dou
             inner->iters = 0;
             inner->err = 0.0;
             inner->converged = 0;
+            inner->pad = 0;
             inner->done = 0;
             if (bb == 0.0) {
                 inner->done = 1;
@@ -1374,9 +1396,10 @@ void launch_refine_sweep(const Operator& op, const double* S64, const float* S32
 }
 
 void launch_refine_check_init(const double* partial, int sweep, double tol, double inner_tol, CgScalars* outer,
-                              CgScalars* inner, int* refine_iters, int nrec, hipStream_t s) {
+                              CgScalars* inner, int* refine_iters, int nrec, unsigned long long* slots,
+                              hipStream_t s) {
     launch_k(refine_check_init_kernel, dim3(1), dim3(kCgThreads), 0, s, partial, sweep, tol, inner_tol, outer, inner,
-             refine_iters, nrec);
+             refine_iters, nrec, slots);
 }
 
 void launch_residual64(const Operator& op, const double* S64, const double* b, const double* dv, int first,

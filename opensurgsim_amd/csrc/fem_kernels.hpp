@@ -43,7 +43,7 @@ struct CgScalars {
                         // one-kernel CG, which writes 2 + k from its launch k (see cg_fused_kernel)
     int converged;
     int iters;          // Eigen's iteration count
-    int pad;
+    int pad;            // 1: a one-launch solve gave up waiting (cg_resident_kernel); cleared by the solve's start
 };
 
 // Staged record sizes (doubles): an off-diagonal block contribution (9 values + pad, so records start on
@@ -170,6 +170,7 @@ struct CgArgs {
     void* w[2] = {nullptr, nullptr};
     double* part7 = nullptr;  // [2][kFusedSums * kCgBlocks], by iteration parity
     void* binv = nullptr;     // FP32 one-kernel iteration: 3x3 block-diagonal preconditioner, 9 floats per node
+    unsigned long long* slots = nullptr;  // one-launch solve: published sums, emptied by the solve's start (or null)
 };
 constexpr int kFusedSums = 7;
 
@@ -214,7 +215,7 @@ void launch_refine_sweep(const Operator& op, const double* S64, const float* S32
                          const double* dv_in, const float* x_in, double* dv_out, int first, float* x_out, float* r,
                          float* z, float* binv, double* partial, const CgScalars* outer, hipStream_t s);
 void launch_refine_check_init(const double* partial, int sweep, double tol, double inner_tol, CgScalars* outer,
-                              CgScalars* inner, int* refine_iters, int nrec, hipStream_t s);
+                              CgScalars* inner, int* refine_iters, int nrec, unsigned long long* slots, hipStream_t s);
 void launch_refine_accumulate(int n, const float* xf, double* dv, const CgScalars* outer, const CgScalars* inner,
                               int* iters_out, hipStream_t s);
 

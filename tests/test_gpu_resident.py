@@ -1,0 +1,156 @@
+"""The one-launch CG (the operator held on the chip) against the CG with one launch per iteration.
+
+Both solve to cg_tolerance TOL = 1e-12, so a step's velocities differ by at most a few TOL times the operator's
+conditioning (dt^2 K / M <= 1e2 at these sizes): 1e-9 in FP64 and with the FP64 refinement around FP32 alike, whose
+outer test is the same. The recurrence is the same, so the iteration counts differ by at most one (the sums are bracketed
+differently) on the block meshes; FP32 inner solves, and the hundreds of iterations that the slivers of a random mesh take,
+follow their own rounding, so their counts are not compared.
+"""
+import functools
+import threading
+
+import numpy as np
+import pytest
+
+from opensurgsim_amd import femgpu
+from opensurgsim_amd import meshgen as mg
+
+pytestmark = pytest.mark.gpu
+TOL, BOUND = 1e-12, 1e-9
+
+
+def block(n):
+    x0, tets, _ = mg.block_tet_mesh(*n)
+    return x0, tets, mg.face_nodes(*n, 1, 0)
+
+
+def irregular(points=900, seed=3):
+    """Delaunay mesh of random points (uneven node degrees) with a node that no element uses."""
+    from scipy.spatial import Delaunay
+    p = np.random.RandomState(seed).rand(points, 3) * 0.1
+    t = Delaunay(p).simplices
+    vol = mg.tet_volumes(p, t)
+    t[vol < 0] = t[vol < 0][:, [0, 1, 3, 2]]
+    t = t[np.abs(vol) > 2e-9]
+    used = np.unique(t)
+    remap = np.full(points, -1)
+    remap[used] = np.arange(used.size)
+    return np.concatenate([p[used], [[0.2, 0.2, 0.2]]]), remap[t].astype(np.int32), np.arange(5)
+
+
+def star(points):
+    """A hub joined to every point of a sphere: one block row of points + 1 blocks, and as many halo columns."""
+    from scipy.spatial import ConvexHull
+    k = np.arange(points) + 0.5
+    ph, th = np.arccos(1 - 2 * k / points), np.pi * (1 + 5 ** 0.5) * k
+    p = 0.1 * np.stack([np.cos(th) * np.sin(ph), np.sin(th) * np.sin(ph), np.cos(ph)], 1)
+    tri = ConvexHull(p).simplices
+    t = np.concatenate([np.full((len(tri), 1), points), tri], 1)
+    x0 = np.concatenate([p, [[0.0, 0.0, 0.0]]])
+    vol = mg.tet_volumes(x0, t)
+    t[vol < 0] = t[vol < 0][:, [0, 1, 3, 2]]
+    return x0, t.astype(np.int32), np.arange(3)
+
+
+def run(mesh, precision, steps=2, **opts):
+    x0, tets, bc = mesh
+    g = femgpu.FemGpu(0)
+    g.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets, 5e4, 0.4, 1000.0)
+    g.add_bc_nodes(bc)
+    g.set_options(**dict(dict(dt=1e-3, cg_tolerance=TOL, precision=precision), **opts))
+    g.set_state(v=0.01 * np.random.RandomState(1).standard_normal(x0.size))
+    its = []
+    for _ in range(steps):
+        assert g.step(1) == femgpu.FEM_OK
+        its.append(g.stats()["last_cg_iterations"])
+    x, v = g.state()
+    conv = g.stats()["converged"]
+    g.close()
+    return x, v, its, conv
+
+
+def both(monkeypatch, mesh, precision, **kw):
+    monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+    a = run(mesh, precision, **kw)
+    monkeypatch.setenv("FEM_CG_KERNELS", "fused")
+    return a, run(mesh, precision, **kw)
+
+
+def same(a, b, precision, counts=True):
+    assert np.linalg.norm(a[1] - b[1]) <= BOUND * np.linalg.norm(b[1])
+    assert np.linalg.norm(a[0] - b[0]) <= BOUND * np.linalg.norm(b[0])
+    if counts and precision == femgpu.FP64:
+        assert all(abs(i - j) <= 1 for i, j in zip(a[2], b[2])), (a[2], b[2])
+    assert a[3] == b[3] == 1
+
+
+# one workgroup, two, an odd count; the fewest and the most blocks per lane; the largest meshes that fit
+@pytest.mark.parametrize("n", [(1, 1, 1), (3, 3, 3), (5, 4, 6), (9, 7, 8), (21, 18, 20), (34, 33, 35), (40, 40, 40)])
+@pytest.mark.parametrize("precision", [femgpu.FP64, femgpu.FP32_REFINED])
+def test_block_meshes(monkeypatch, n, precision):
+    a, b = both(monkeypatch, block(n), precision)
+    same(a, b, precision)
+
+
+@pytest.mark.parametrize("precision", [femgpu.FP64, femgpu.FP32_REFINED])
+def test_beyond_the_chip_and_largest_fp32(monkeypatch, precision):
+    a, b = both(monkeypatch, block((50, 48, 49)), precision, steps=1)
+    same(a, b, precision)
+
+
+# FP32 CG does not converge on the random mesh's slivers, with either CG: FP64 alone there
+@pytest.mark.parametrize("mesh, precision", [(irregular, femgpu.FP64)] + [
+    (functools.partial(star, n), p) for n in (700, 1500) for p in (femgpu.FP64, femgpu.FP32_REFINED)])
+def test_uneven_rows(monkeypatch, mesh, precision):
+    a, b = both(monkeypatch, mesh(), precision)
+    same(a, b, precision, counts=False)
+
+
+@pytest.mark.parametrize("cap", [1, 2, 5])
+def test_iteration_cap(monkeypatch, cap):
+    a, b = both(monkeypatch, block((6, 7, 5)), femgpu.FP64, cg_max_iterations=cap, steps=1)
+    assert a[2] == b[2] == [cap] and a[3] == b[3] == 0
+    assert np.linalg.norm(a[1] - b[1]) <= 1e-12 * np.linalg.norm(b[1])
+
+
+def test_zero_right_hand_side():
+    x0, tets, bc = block((3, 3, 3))
+    g = femgpu.FemGpu(0)
+    g.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets, 5e4, 0.4, 1000.0)
+    g.add_bc_nodes(bc)
+    g.set_options(dt=1e-3, cg_tolerance=TOL, gravity_enabled=0)
+    for _ in range(3):
+        assert g.step(1) == femgpu.FEM_OK
+    x, v = g.state()
+    assert g.stats()["last_cg_iterations"] == 0 and not v.any() and np.array_equal(x, x0.reshape(-1))
+    g.close()
+
+
+@pytest.mark.parametrize("precision", [femgpu.FP64, femgpu.FP32_REFINED])
+def test_gives_up_waiting_and_solves_anyway(monkeypatch, precision):
+    """No wait is allowed: the first one gives up, and the solve goes on with one launch per iteration."""
+    mesh = block((12, 11, 13))
+    monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+    monkeypatch.setenv("FEM_CG_WAIT_US", "0")
+    a = run(mesh, precision, steps=3)
+    monkeypatch.delenv("FEM_CG_WAIT_US")
+    b = run(mesh, precision, steps=3)
+    same(a, b, precision)
+
+
+def test_repeats_bit_for_bit_and_from_threads(monkeypatch):
+    monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+    meshes = [block((12, 11, 13)), block((21, 18, 20))]
+    want = [run(m, femgpu.FP64, steps=6) for m in meshes]
+    got = [None, None]
+
+    def work(i):
+        got[i] = run(meshes[i], femgpu.FP64, steps=6)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(60)
+    for w, g in zip(want, got):
+        assert np.array_equal(w[0], g[0]) and np.array_equal(w[1], g[1])
