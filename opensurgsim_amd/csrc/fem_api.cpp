@@ -242,6 +242,11 @@ struct fem_ctx {
     DevBuf<double> part7;      // [2][kFusedSums * kCgBlocks] block sums of the fused CG kernel, by parity
     // one-launch CG solves (fem_resident.hip): the partition for res_precision, exchanged vectors, published sums
     ResidentTables res;
+    std::vector<int> res_launches;        // batch: workgroups of each launch
+    std::vector<uint8_t> res_instances;   // batch: the instances these solve
+    int res_columns = 1;                  // columns that fit one launch
+    DevBuf<double> res_col;               // their r, z, preconditioner and partial sums
+    DevBuf<CgScalars> res_col_sc;
     int res_precision = -1;
     std::vector<double> h_x0;  // rest positions, for the partition
     bool res_dirty = false;    // the exchanged vectors have to be emptied (new, or left by a solve that gave up)
@@ -495,9 +500,13 @@ void ensure_resident(fem_ctx* c, bool fp32) {
     if (c->res_precision == (fp32 ? 1 : 0)) return;
     c->res = ResidentTables{};
     c->res_precision = fp32 ? 1 : 0;
-    if (c->cg_kernels != 0 || c->kind == FEM_ELEMENT_HEX || c->num_instances > 0) return;
-    const ResidentPlan plan = plan_resident(c->num_nodes, c->h_rowptr_b.data(), c->h_colidx_b.data(), c->h_x0.data(),
-                                            fp32, c->num_cus);
+    c->res_columns = 1;
+    if (c->cg_kernels != 0 || c->kind == FEM_ELEMENT_HEX) return;
+    const ResidentPlan plan =
+        c->num_instances > 0 ? plan_resident_batch(c->h_node_off, c->h_rowptr_b.data(), c->h_colidx_b.data(),
+                                                   c->h_x0.data(), fp32, c->num_cus)
+                             : plan_resident(c->num_nodes, c->h_rowptr_b.data(), c->h_colidx_b.data(), c->h_x0.data(),
+                                             fp32, c->num_cus);
     if (plan.groups == 0) return;
     std::vector<unsigned char> h;
     std::vector<size_t> at;
@@ -515,15 +524,21 @@ void ensure_resident(fem_ctx* c, bool fp32) {
     add(plan.lane_info);
     add(plan.row_lane);
     add(plan.cols);
+    add(plan.wg);
     c->res_mem.alloc(h.size());
     c->res_mem.upload(h.data(), h.size(), c->stream);
-    c->res_exch.alloc(2 * (size_t)c->num_nodes * (fp32 ? kResRowBytes32 : kResRowBytes64));
+    // columns of a compliance solve (FP64) go side by side while CUs are left
+    if (c->num_instances == 0 && !fp32)
+        c->res_columns = std::max(1, std::min(kResMaxColumns, std::min(c->num_cus, kResMaxGroups) / plan.groups));
+    c->res_exch.alloc(2 * (size_t)c->res_columns * c->num_nodes * (fp32 ? kResRowBytes32 : kResRowBytes64));
     c->res_dirty = true;
-    if (!c->res_slots.p) c->res_slots.alloc(kResSlotWords);
+    c->res_slots.alloc(kResSlotWords * std::max<size_t>(1, plan.launches.size()));
+    c->res_launches = plan.launches;
+    c->res_instances = plan.instances;
     HIPCHECK(hipStreamSynchronize(c->stream));
     unsigned char* p = c->res_mem.p;
     c->res.nb = plan.nb;
-    c->res.max_cols = plan.max_cols;
+    c->res.rows = (int)c->num_nodes;
     c->res.group = reinterpret_cast<const int4*>(p + at[0]);
     c->res.row_node = reinterpret_cast<const int*>(p + at[1]);
     c->res.halo_node = reinterpret_cast<const int*>(p + at[2]);
@@ -532,12 +547,15 @@ void ensure_resident(fem_ctx* c, bool fp32) {
     c->res.lane_info = reinterpret_cast<const int*>(p + at[5]);
     c->res.row_lane = reinterpret_cast<const uint16_t*>(p + at[6]);
     c->res.cols = reinterpret_cast<const uint16_t*>(p + at[7]);
+    c->res.wg = c->num_instances > 0 ? reinterpret_cast<const int4*>(p + at[8]) : nullptr;
     c->res.groups = plan.groups;
 }
 
 bool use_resident(const fem_ctx* c, bool fp32) {
     return c->res.groups > 0 && c->res_precision == (fp32 ? 1 : 0) && c->res_backoff == 0;
 }
+
+constexpr int kResBackoff = 256;  // solves with one launch per iteration after a one-launch solve gave up
 
 // One-launch solves of a device go one after another: two of them side by side could each hold CUs that the other's
 // workgroups wait for. Held from the launch until the host has seen the solve's end.
@@ -546,23 +564,28 @@ std::mutex& resident_mutex(int device) {
     return mu[(unsigned)device % 64];
 }
 
-void launch_resident(fem_ctx* c, const CgArgs& a, int max_iter) {
+ResidentArgs resident_args(fem_ctx* c) {
     if (c->res_dirty) {
         HIPCHECK(hipMemsetAsync(c->res_exch.p, 0, c->res_exch.n, c->stream));
         c->res_dirty = false;
     }
     ResidentArgs r;
     r.t = c->res;
+    r.exch = c->res_exch.p;
+    r.slots = c->res_slots.p;
+    r.wait_ticks = c->res_wait_ticks;
+    return r;
+}
+
+void launch_resident(fem_ctx* c, const CgArgs& a, int max_iter) {
+    ResidentArgs r = resident_args(c);
     r.S = a.S;
     r.r = a.r1;
     r.z = a.z1;
     r.x = a.x;
     r.dinv = a.fp32 ? a.binv : a.dinv;
-    r.exch = c->res_exch.p;
-    r.slots = c->res_slots.p;
     r.sc = a.sc;
     r.max_iter = max_iter;
-    r.wait_ticks = c->res_wait_ticks;
     launch_cg_resident(r, a.fp32, c->stream);
 }
 
@@ -631,8 +654,6 @@ int64_t max_iters(fem_ctx* c) {
     int64_t m = c->opt.cg_max_iterations < 0 ? 2 * c->ndof : c->opt.cg_max_iterations;
     return std::min<int64_t>(m, std::numeric_limits<int>::max() - 1);
 }
-
-constexpr int kResBackoff = 256;  // solves with one launch per iteration after a one-launch solve gave up
 
 // Runs the CG iterations of an initialised solve of right-hand side b: in one launch where the operator fits the
 // chip (a.slots), otherwise launches a predicted number of iterations, then polls the device 'done' flag between
@@ -1248,6 +1269,10 @@ BatchCg batch_args(fem_ctx* c, bool fp32) {
     a.sc = c->b_sc.p;
     a.kA = c->b_kA.p;
     a.kV = c->b_kV.p;
+    if (use_resident(c, fp32) && c->opt.cg_max_iterations != 0) {
+        a.slots = c->res_slots.p;
+        a.slot_words = c->res_slots.n;
+    }
     return a;
 }
 
@@ -1323,6 +1348,51 @@ int run_batch_iterations(fem_ctx* c, const BatchCg& a, int& predicted) {
     return mx;
 }
 
+// The solves that launch_batch_cg_init(a, b, skip, tol) has started: in one launch each for the instances that the
+// partition takes, the others by iterations over the chunks. Returns the largest iteration count.
+int run_batch_solves(fem_ctx* c, const BatchCg& a, const double* b, const CgScalars* skip, double tol, int& predicted) {
+    if (!a.slots) return run_batch_iterations(c, a, predicted);
+    const int M = c->num_instances;
+    bool gave_up = false, rest = false;
+    {
+        std::lock_guard<std::mutex> one(resident_mutex(c->device));
+        ResidentArgs r = resident_args(c);
+        r.S = a.S;
+        r.r = a.r;
+        r.z = a.z;
+        r.x = a.x;
+        r.dinv = a.dinv;
+        r.sc = a.sc;
+        r.max_iter = 0;
+        r.max_iters = a.t.inst_maxit;
+        for (int wgs : c->res_launches) {
+            launch_cg_resident(r, a.fp32, c->stream, wgs);
+            r.t.wg += wgs;
+            r.slots += kResSlotWords;
+        }
+        HIPCHECK(hipMemcpyAsync(c->h_bsc, a.sc, M * sizeof(CgScalars), hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(hipStreamSynchronize(c->stream));
+    }
+    int mx = 0;
+    for (int i = 0; i < M; ++i) {
+        gave_up = gave_up || c->h_bsc[i].pad;
+        rest = rest || (!c->res_instances[i] && !c->h_bsc[i].done);
+        mx = std::max(mx, c->h_bsc[i].iters);
+    }
+    if (gave_up) {
+        c->res_backoff = kResBackoff;
+        c->res_dirty = true;
+        BatchCg t = a;
+        t.slots = nullptr;
+        t.slot_words = 0;
+        launch_batch_cg_init(t, b, skip, tol, c->b_lanes, c->stream);
+        return run_batch_iterations(c, t, predicted);
+    }
+    if (rest) return run_batch_iterations(c, a, predicted);
+    predicted = mx + 1;
+    return mx;
+}
+
 // Autotuner: time CG iterations over all chunks for each (chunk rows, lanes per row) on the current operator and
 // rhs. Shapes within 2 % of the fastest are taken as tied (run to run, close shapes swap places), and the tie goes
 // to the fewest rows per chunk, then the fewest lanes per row: once a few long solves remain, their iterations go
@@ -1383,11 +1453,13 @@ void batch_linear_solve(fem_ctx* c) {
     const int M = c->num_instances;
     refresh_batch_params(c);
     if (!c->b_tuned) tune_batch(c, fp32);
+    ensure_resident(c, fp32);
+    if (c->res_backoff > 0) --c->res_backoff;
     std::fill(c->h_inst_iters.begin(), c->h_inst_iters.end(), 0);
     if (!fp32) {
         BatchCg a = batch_args(c, false);
         launch_batch_cg_init(a, c->b.p, nullptr, c->opt.cg_tolerance, c->b_lanes, c->stream);
-        const int it = run_batch_iterations(c, a, c->b_predicted[0]);
+        const int it = run_batch_solves(c, a, c->b.p, nullptr, c->opt.cg_tolerance, c->b_predicted[0]);
         int64_t total = 0;
         bool conv = true;
         double err = 0.0;
@@ -1418,7 +1490,7 @@ void batch_linear_solve(fem_ctx* c) {
         if (sweep == c->opt.max_refinements) break;
         launch_batch_cg_init(a, c->r64.p, c->b_outer.p, c->opt.inner_tolerance, c->b_lanes, c->stream);
         int& pred = c->b_predicted[1 + std::min(sweep, 15)];
-        longest += run_batch_iterations(c, a, pred) + 1;
+        longest += run_batch_solves(c, a, c->r64.p, c->b_outer.p, c->opt.inner_tolerance, pred) + 1;
         for (int i = 0; i < M; ++i)
             if (!c->h_bsc[i].converged || c->h_bsc[i].iters > 0) {
                 c->h_inst_iters[i] += c->h_bsc[i].iters;
@@ -2441,6 +2513,63 @@ void mcg_columns(fem_ctx* c, const double* b, int64_t ncols, double* out, const 
     }
 }
 
+// Work vectors of the one-launch column solves: r and z of the columns of a launch, the preconditioner, partial sums,
+// and the scalars of kResColumnStates columns.
+constexpr int kResColumnStates = 256;
+struct ColumnWork {
+    double *r, *z, *dinv, *partial;
+    CgScalars* sc;
+};
+size_t column_work_doubles(size_t n, int columns) {
+    return (2 * (size_t)columns + 1) * n + 2 * (size_t)kResColumnBlocks * columns;
+}
+ColumnWork column_work(double* base, CgScalars* sc, size_t n, int columns) {
+    return {base, base + columns * n, base + 2 * columns * n, base + (2 * columns + 1) * n, sc};
+}
+
+// Columns [0, ncols) of b through the one-launch CG, c->res_columns side by side; x is written in place in out, with the
+// boundary rows zero from the start. False when a solve gave up waiting (out is then solved again by the caller).
+bool resident_columns(fem_ctx* c, const double* b, int64_t ncols, double* out, const ColumnWork& w) {
+    const size_t n = (size_t)c->ndof;
+    CgScalars h[kResColumnStates];
+    std::lock_guard<std::mutex> one(resident_mutex(c->device));
+    for (int64_t j0 = 0; j0 < ncols; j0 += kResColumnStates) {
+        const int some = (int)std::min<int64_t>(kResColumnStates, ncols - j0);
+        for (int j = 0; j < some; j += c->res_columns) {
+            const int cnt = std::min(c->res_columns, some - j);
+            ResidentArgs r = resident_args(c);
+            r.S = c->S64.p;
+            r.r = w.r;
+            r.z = w.z;
+            r.x = out + (j0 + j) * n;
+            r.dinv = w.dinv;
+            r.sc = w.sc + j;
+            r.max_iter = (int)max_iters(c);
+            r.solves = cnt;
+            r.stride = (int64_t)n;
+            launch_resident_columns((int)c->num_nodes, cnt, b + (j0 + j) * n, c->bcmask.p, c->diagblk.p, c->S64.p,
+                                    c->opt.cg_tolerance, out + (j0 + j) * n, w.r, w.z, w.dinv, w.partial, w.sc + j,
+                                    c->res_slots.p, c->stream);
+            launch_cg_resident(r, false, c->stream);
+        }
+        HIPCHECK(hipMemcpyAsync(h, w.sc, some * sizeof(CgScalars), hipMemcpyDeviceToHost, c->stream));
+        HIPCHECK(hipStreamSynchronize(c->stream));
+        for (int j = 0; j < some; ++j)
+            if (h[j].pad) {
+                c->res_backoff = kResBackoff;
+                c->res_dirty = true;
+                return false;
+            }
+    }
+    return true;
+}
+
+// Whether compliance columns take the one-launch CG: b and out apart (a solve that gives up starts again from b).
+bool use_resident_columns(fem_ctx* c, const double* b, const double* out, int64_t ncols) {
+    const int64_t len = ncols * c->ndof;
+    return use_resident(c, false) && c->num_instances == 0 && max_iters(c) >= 1 && (b + len <= out || out + len <= b);
+}
+
 // Compliance columns through the band LU (LinearSparseSolveAndInverseLU::solve): each column of b with its
 // boundary rows zeroed into tmp (tmp_cols columns of ndof at a time), solved into out, boundary rows of the
 // solutions zeroed (DeformableRepresentation::applyCompliance, Physics/DeformableRepresentation.cpp:175-190).
@@ -2475,6 +2604,12 @@ void compliance_tet(fem_ctx* c, const double* b, int64_t ncols, double* out) {
             for (int64_t j = full; j < ncols; ++j) compliance_column(c, b + (size_t)j * n, out + (size_t)j * n);
             ncols = full;
         }
+    }
+    if (use_resident_columns(c, b, out, ncols)) {
+        const size_t need = column_work_doubles(n, c->res_columns);
+        if (c->res_col.n < need) c->res_col.alloc(need);
+        if (!c->res_col_sc.p) c->res_col_sc.alloc(kResColumnStates);
+        if (resident_columns(c, b, ncols, out, column_work(c->res_col.p, c->res_col_sc.p, n, c->res_columns))) return;
     }
     if (c->mcg_b.n != n * 8) {
         for (DevBuf<double>* v : {&c->mcg_b, &c->mcg_x, &c->mcg_r, &c->mcg_z, &c->mcg_p, &c->mcg_q}) v->alloc(n * 8);
@@ -2573,6 +2708,12 @@ int fem_apply_compliance_device_noalloc(fem_ctx* c, const double* b, int64_t num
             compliance_lu(c, b, num_columns, out, (double*)base, tc);
             return FEM_OK;
         }
+        const size_t work = column_work_doubles((size_t)c->ndof, c->res_columns) * sizeof(double);
+        const size_t work_up = (work + 255) & ~size_t(255);
+        if (use_resident_columns(c, b, out, num_columns) && work_up + kResColumnStates * sizeof(CgScalars) <= kNoAllocScratchBytes &&
+            resident_columns(c, b, num_columns, out,
+                             column_work((double*)base, (CgScalars*)(base + work_up), (size_t)c->ndof, c->res_columns)))
+            return FEM_OK;
         McgColumn status[8];
         const McgWork w{(double*)(base + L.b), (double*)(base + L.x), (double*)(base + L.r),
                         (double*)(base + L.z), (double*)(base + L.p), (double*)(base + L.q),
@@ -2989,6 +3130,8 @@ int fem_set_instances(fem_ctx* c, int32_t num_instances, const int64_t* node_off
             ei[e] = i;
         }
         c->num_instances = M;
+        c->res_precision = -1;  // planned per instance at the next solve
+        c->res = ResidentTables{};
         c->linear_matrix_ready = false;
         c->elem_inst.alloc(c->num_elements);
         c->elem_inst.upload(ei.data(), c->num_elements, c->stream);

@@ -7,6 +7,7 @@
 #include "fem_batch.hpp"
 #include "fem_device.hpp"
 #include "fem_reduce.hpp"
+#include "fem_resident.hpp"
 
 #include <cfloat>
 
@@ -126,9 +127,13 @@ __global__ __launch_bounds__(kBatchThreads) void bcg_init_kernel(BatchTables t, 
 // One workgroup per instance.
 __global__ __launch_bounds__(kBatchThreads) void bcg_init2_kernel(BatchTables t, const double* __restrict__ partial,
                                                                   CgScalars* sc, const CgScalars* __restrict__ skip,
-                                                                  double tol, int* kA, int* kV) {
+                                                                  double tol, int* kA, int* kV,
+                                                                  unsigned long long* __restrict__ slots,
+                                                                  size_t slot_words) {
     __shared__ double lds[64];
     const int inst = blockIdx.x;
+    for (size_t i = inst * (size_t)blockDim.x + threadIdx.x; i < slot_words; i += gridDim.x * (size_t)blockDim.x)
+        slots[i] = kResEmpty;
     if (threadIdx.x == 0) {
         kA[inst] = 0;
         kV[inst] = 0;
@@ -411,7 +416,7 @@ void launch_batch_cg_init(const BatchCg& a, const double* b, const CgScalars* sk
         launch_k((bcg_init_kernel<double>), grid, block, 0, s, a.t, a.op, (const double*)a.S, b, (double*)a.x,
                  (double*)a.r, (double*)a.z, (double*)a.dinv, a.partial, skip);
     launch_k(bcg_init2_kernel, dim3(a.t.num_instances), block, 0, s, a.t, (const double*)a.partial, a.sc, skip, tol,
-             a.kA, a.kV);
+             a.kA, a.kV, a.slots, a.slot_words);
 }
 
 void launch_batch_cg_iteration(const BatchCg& a, int lanes, hipStream_t s) {

@@ -48,6 +48,8 @@ struct BatchCg {
     CgScalars* sc;     // [M] inner
     int* kA;           // [M]
     int* kV;           // [M]
+    unsigned long long* slots = nullptr;  // one-launch solves: published words, emptied by the init (or null)
+    size_t slot_words = 0;
 };
 
 // x = 0, r = b, dinv, z, per-instance |b|^2 and r.z; instances whose skip[i].done is set are left alone.

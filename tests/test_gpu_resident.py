@@ -154,3 +154,74 @@ def test_repeats_bit_for_bit_and_from_threads(monkeypatch):
         t.join(60)
     for w, g in zip(want, got):
         assert np.array_equal(w[0], g[0]) and np.array_equal(w[1], g[1])
+
+
+def run_batch(sizes, precision, steps=2):
+    off, parts = [0], []
+    for n in sizes:
+        x0, tets, bc = block(n)
+        parts.append((x0, tets + off[-1], bc + off[-1]))
+        off.append(off[-1] + len(x0))
+    x0, tets, bc = (np.concatenate([p[i] for p in parts]) for i in range(3))
+    g = femgpu.FemGpu(0)
+    g.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets.astype(np.int32), 5e4, 0.4, 1000.0)
+    g.add_bc_nodes(bc)
+    g.set_batch_tuning(128, 8)
+    g.set_instances(off, np.resize([5e-4, 1e-3, 2e-3], len(sizes)))
+    g.set_options(dt=1e-3, cg_tolerance=TOL, precision=precision)
+    g.set_state(v=0.01 * np.random.RandomState(1).standard_normal(x0.size))
+    assert g.step(steps) == femgpu.FEM_OK
+    x, v = g.state()
+    its, _, conv = g.instance_stats()
+    g.close()
+    return x, v, its, conv
+
+
+# one instance, uneven ones in one launch, more than one launch holds, and one that does not fit beside others that do
+@pytest.mark.parametrize("sizes", [[(4, 5, 3)], [(3, 3, 3), (9, 8, 7), (14, 3, 6), (6, 6, 6), (20, 18, 19)],
+                                   [(10, 9, 11)] * 70, [(48, 50, 49), (5, 5, 5), (12, 9, 10)]],
+                         ids=["one", "uneven", "launches", "oversize"])
+@pytest.mark.parametrize("precision", [femgpu.FP64, femgpu.FP32_REFINED])
+def test_batches(monkeypatch, sizes, precision):
+    monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+    a = run_batch(sizes, precision)
+    monkeypatch.setenv("FEM_CG_KERNELS", "fused")
+    b = run_batch(sizes, precision)
+    for i in (0, 1):
+        assert np.linalg.norm(a[i] - b[i]) <= BOUND * np.linalg.norm(b[i])
+    assert a[3].all() and b[3].all()
+    if precision == femgpu.FP64:
+        assert np.abs(a[2] - b[2]).max() <= 1
+
+
+def test_batch_gives_up_waiting(monkeypatch):
+    sizes = [(6, 7, 5), (9, 8, 7)]
+    monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+    b = run_batch(sizes, femgpu.FP64)
+    monkeypatch.setenv("FEM_CG_WAIT_US", "0")
+    a = run_batch(sizes, femgpu.FP64)
+    assert np.linalg.norm(a[1] - b[1]) <= BOUND * np.linalg.norm(b[1])
+
+
+# fewer columns than fit side by side, more, and a mesh that takes the chip alone; a zero column among them
+@pytest.mark.parametrize("n, columns", [((3, 4, 3), 1), ((3, 4, 3), 70), ((12, 11, 13), 11), ((34, 33, 35), 3)])
+@pytest.mark.parametrize("wait", [None, "0"])
+def test_compliance_columns(monkeypatch, n, columns, wait):
+    x0, tets, bc = block(n)
+    B = np.random.RandomState(2).standard_normal((x0.size, columns))
+    B[:, columns // 2] = 0.0 if columns > 1 else B[:, 0]
+    got = []
+    for env in (None, "fused"):
+        monkeypatch.setenv("FEM_CG_KERNELS", env) if env else monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+        monkeypatch.setenv("FEM_CG_WAIT_US", wait) if wait else monkeypatch.delenv("FEM_CG_WAIT_US", raising=False)
+        g = femgpu.FemGpu(0)
+        g.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets, 5e4, 0.4, 1000.0)
+        g.add_bc_nodes(bc)
+        g.set_options(dt=1e-3, cg_tolerance=TOL)
+        assert g.step(1) == femgpu.FEM_OK
+        got.append(g.apply_compliance(B))
+        g.close()
+    for j in range(columns):
+        assert np.linalg.norm(got[0][:, j] - got[1][:, j]) <= BOUND * np.linalg.norm(got[1][:, j])
+    for node in bc:
+        assert not got[0][3 * node:3 * node + 3].any()
