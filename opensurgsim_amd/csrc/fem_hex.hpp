@@ -26,6 +26,9 @@ struct HexData {
     int* order = nullptr;         // elements sorted by color
     std::vector<int> pad_ptr;     // colour c: order_pad[pad_ptr[c] .. pad_ptr[c + 1]), multiples of 64
     int* order_pad = nullptr;     // colour order padded to 64-element tiles (-1 = padding)
+    void* stage = nullptr;        // staged products of an application, 24 values per padded position (see fem_hex.hip)
+    int* src = nullptr;           // [slots][num_nodes] where each node's values are staged, colour order (-1: none)
+    int slots = 0;                // most elements of a node
     float* A32 = nullptr;         // packed upper triangle of M/dt + dt K (FP32): 28 upper node blocks of 9 and
                                   // 8 symmetric diagonal blocks of 6, 300 floats per padded position,
                                   // interleaved by 64-position tiles in float4 chunks
