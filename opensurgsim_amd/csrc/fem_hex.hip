@@ -97,22 +97,21 @@ constexpr int kHexChunks = 75;
 constexpr int kHexOffFloats = 252;
 constexpr int kHexMaxDistinct = 32;  // distinct-matrix table: at most 38.4 KB of LDS per workgroup
 
-// Strictly upper node block o (0..27) of the packed order: its nodes (a, b), a < b.
-__host__ __device__ constexpr int off_a(int o) {
-    int a = 0;
-    while (o >= 7 - a) {
-        o -= 7 - a;
-        ++a;
-    }
-    return a;
-}
-__host__ __device__ constexpr int off_b(int o) {
-    int a = 0;
-    while (o >= 7 - a) {
-        o -= 7 - a;
-        ++a;
-    }
-    return a + 1 + o;
+// Strictly upper node block o (0..27) of the packed order: its nodes (a, b), a < b. A table: computed by a loop in the
+// unrolled products, the nodes were not constants to the compiler, which then indexed the registers at run time (274
+// s_set_gpr_idx and as many moves per element, 9.5 us of a 17 us application on 64x33x65 cubes).
+struct OffBlocks {
+    int a[28], b[28];
+};
+__host__ __device__ constexpr OffBlocks off_blocks() {
+    OffBlocks t = {};
+    int o = 0;
+    for (int a = 0; a < 8; ++a)
+        for (int b = a + 1; b < 8; ++b, ++o) {
+            t.a[o] = a;
+            t.b[o] = b;
+        }
+    return t;
 }
 __host__ __device__ constexpr int off_index(int a, int b) { return 7 * a - a * (a - 1) / 2 + (b - a - 1); }
 // Packed float of entry (i, j) of a diagonal block (upper triangle, i <= j).
@@ -162,35 +161,35 @@ __global__ __launch_bounds__(256) void hex_prepare_kernel(int count_pad, const i
     }
 }
 
-// FP64 element operator y = alpha_m M pm + alpha_k K p for one element (matrix-free; lumped: M's row
-// sums on the diagonal).
-__device__ __forceinline__ void hex_apply64(const double* X, const double4 m, const double* p, const double* pm,
-                                            double am, double ak, int lumped, double* y) {
-    for (int i = 0; i < 24; ++i) y[i] = 0.0;
-    for (int gi = 0; gi < 2; ++gi)
-        for (int gj = 0; gj < 2; ++gj)
-            for (int gk = 0; gk < 2; ++gk) {
-                double N[8], g[8][3];
-                const double w = hex_gp(X, gi, gj, gk, N, g);
-                double H[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-                double np[3] = {0, 0, 0};
-                for (int b = 0; b < 8; ++b)
-                    for (int i = 0; i < 3; ++i) {
-                        np[i] += N[b] * pm[3 * b + i];
-                        for (int j = 0; j < 3; ++j) H[3 * i + j] += p[3 * b + i] * g[b][j];
-                    }
-                const double sn = ((N[0] + N[1]) + (N[2] + N[3])) + ((N[4] + N[5]) + (N[6] + N[7]));
-                const double tr = H[0] + H[4] + H[8];
-                double sig[9];
-                for (int i = 0; i < 3; ++i)
-                    for (int j = 0; j < 3; ++j)
-                        sig[3 * i + j] = m.y * (H[3 * i + j] + H[3 * j + i]) + (i == j ? m.x * tr : 0.0);
-                const double wk = ak * w, wm = am * w * m.z;
-                for (int a = 0; a < 8; ++a)
-                    for (int i = 0; i < 3; ++i)
-                        y[3 * a + i] += wk * (sig[3 * i] * g[a][0] + sig[3 * i + 1] * g[a][1] + sig[3 * i + 2] * g[a][2]) +
-                                        wm * N[a] * (lumped ? sn * pm[3 * a + i] : np[i]);
+// FP64 element operator y += (alpha_m M + alpha_k K) p for one element (matrix-free; lumped: M's row
+// sums on the diagonal). The Gauss points stay a loop: unrolled, the lane held over 256 registers and one wave ran on
+// a SIMD.
+__device__ __forceinline__ void hex_apply64(const double* X, const double4 m, const double* p, double am, double ak,
+                                            int lumped, double* y) {
+#pragma unroll 1
+    for (int gp = 0; gp < 8; ++gp) {
+        const int gi = gp >> 2, gj = (gp >> 1) & 1, gk = gp & 1;
+        double N[8], g[8][3];
+        const double w = hex_gp(X, gi, gj, gk, N, g);
+        double H[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+        double np[3] = {0, 0, 0};
+        for (int b = 0; b < 8; ++b)
+            for (int i = 0; i < 3; ++i) {
+                np[i] += N[b] * p[3 * b + i];
+                for (int j = 0; j < 3; ++j) H[3 * i + j] += p[3 * b + i] * g[b][j];
             }
+        const double sn = ((N[0] + N[1]) + (N[2] + N[3])) + ((N[4] + N[5]) + (N[6] + N[7]));
+        const double tr = H[0] + H[4] + H[8];
+        double sig[9];
+        for (int i = 0; i < 3; ++i)
+            for (int j = 0; j < 3; ++j)
+                sig[3 * i + j] = m.y * (H[3 * i + j] + H[3 * j + i]) + (i == j ? m.x * tr : 0.0);
+        const double wk = ak * w, wm = am * w * m.z;
+        for (int a = 0; a < 8; ++a)
+            for (int i = 0; i < 3; ++i)
+                y[3 * a + i] += wk * (sig[3 * i] * g[a][0] + sig[3 * i + 1] * g[a][1] + sig[3 * i + 2] * g[a][2]) +
+                                wm * N[a] * (lumped ? sn * p[3 * a + i] : np[i]);
+    }
 }
 
 // The staged products: position t of the padded colour order (tile t / 64, lane t % 64) keeps value j of its 24 at
@@ -198,37 +197,65 @@ __device__ __forceinline__ void hex_apply64(const double* X, const double4 m, co
 __device__ __forceinline__ size_t stage_at(int t) { return (size_t)(t >> 6) * 24 * 64 + (t & 63); }
 
 // Convergence test of iteration k - 1 and beta of iteration k (Eigen's recurrence), at the start of the iteration's element
-// kernel; every thread calls it, workgroup 0 records the scalars. False: the solve has ended.
-__device__ __forceinline__ bool hex_cg_begin(int k, int max_iter, const double* partial, CgScalars* sc, double& beta,
-                                             double* lds) {
-    beta = 0.0;
-    if (k <= 0) return true;
-    double rr, rzk;
-    reduce_partials2(partial, partial + kCgBlocks, rr, rzk, lds);
-    const bool first = blockIdx.x == 0 && threadIdx.x == 0;
-    if (rr < sc->threshold || k >= max_iter) {
-        if (first) {
-            const bool conv = rr < sc->threshold;
-            sc->rr = rr;
-            sc->err = sqrt(rr / sc->bb);
-            sc->iters = conv ? k - 1 : k;
-            sc->converged = conv ? 1 : 0;
-            sc->done = 1;
+// kernel, in two parts: the block sums |r|^2 and r.z of the last vector kernel are asked for (wave 0), then added up in a fixed
+// order and used. Every thread calls both; workgroup 0 records the scalars.
+struct HexCgStart {
+    static constexpr int kPer = kCgBlocks / 64;
+    double a[kPer], b[kPer];
+    __device__ __forceinline__ HexCgStart(int k, const double* partial) {
+        if (k > 0 && threadIdx.x < 64) {
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                a[q] = partial[threadIdx.x + 64 * q];
+                b[q] = partial[kCgBlocks + threadIdx.x + 64 * q];
+            }
         }
-        return false;
     }
-    beta = rzk / sc->rz[(k - 1) & 1];
-    if (first) {
-        sc->rz[k & 1] = rzk;
-        sc->rr = rr;
+    // False: the solve has ended. Ends with a barrier for k > 0.
+    __device__ __forceinline__ bool finish(int k, int max_iter, CgScalars* sc, double& beta, double* lds) {
+        beta = 0.0;
+        if (k <= 0) return true;
+        if (threadIdx.x < 64) {
+            double va = 0.0, vb = 0.0;
+#pragma unroll
+            for (int q = 0; q < kPer; ++q) {
+                va += a[q];
+                vb += b[q];
+            }
+            va = wave_total(va);
+            vb = wave_total(vb);
+            if (threadIdx.x == 0) {
+                lds[0] = va;
+                lds[1] = vb;
+            }
+        }
+        __syncthreads();
+        const double rr = lds[0], rzk = lds[1];
+        const bool first = blockIdx.x == 0 && threadIdx.x == 0;
+        if (rr < sc->threshold || k >= max_iter) {
+            if (first) {
+                const bool conv = rr < sc->threshold;
+                sc->rr = rr;
+                sc->err = sqrt(rr / sc->bb);
+                sc->iters = conv ? k - 1 : k;
+                sc->converged = conv ? 1 : 0;
+                sc->done = 1;
+            }
+            return false;
+        }
+        beta = rzk / sc->rz[(k - 1) & 1];
+        if (first) {
+            sc->rz[k & 1] = rzk;
+            sc->rr = rr;
+        }
+        return true;
     }
-    return true;
-}
+};
 
 // stage = (alpha_m M + alpha_k K) w_e of every element. RHS: K acts on w = (x - x0) + kv v and M on v. Otherwise w = p (zero on
 // BC DOFs when mask != null), or with sc != null w = z + beta p of CG iteration k.
 template <bool RHS>
-__global__ __launch_bounds__(128) void hex_apply64_kernel(int count_pad, const int* __restrict__ order_pad,
+__global__ __launch_bounds__(128, 2) void hex_apply64_kernel(int count_pad, const int* __restrict__ order_pad,
                                                           const int* __restrict__ conn, const double* __restrict__ x0,
                                                           const double4* __restrict__ mat, const double* __restrict__ p,
                                                           const double* __restrict__ xcur, const double* __restrict__ v,
@@ -237,30 +264,37 @@ __global__ __launch_bounds__(128) void hex_apply64_kernel(int count_pad, const i
                                                           int max_iter, const double* __restrict__ z,
                                                           const double* __restrict__ partial, CgScalars* sc) {
     __shared__ double lds[64];
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = t < count_pad ? order_pad[t] : -1;
+    HexCgStart start(sc ? k : 0, partial);
     if (sc && sc->done) return;
     double beta = 0.0;
-    if (sc && !hex_cg_begin(k, max_iter, partial, sc, beta, lds)) return;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= count_pad) return;
-    const int e = order_pad[t];
+    if (sc && !start.finish(k, max_iter, sc, beta, lds)) return;
     if (e < 0) return;
-    double X[24], w[24], wm[24], out[24];
+    double X[24], w[24], out[24];
+#pragma unroll
     for (int i = 0; i < 8; ++i) {
         const int id = conn[8 * e + i];
+#pragma unroll
         for (int c = 0; c < 3; ++c) {
             const size_t d = 3 * (size_t)id + c;
             X[3 * i + c] = x0[d];
-            if (RHS) {
-                w[3 * i + c] = (xcur[d] - x0[d]) + kv * v[d];
-                wm[3 * i + c] = v[d];
-            } else if (sc) {
-                w[3 * i + c] = k > 0 ? z[d] + beta * p[d] : z[d];
-            } else {
-                w[3 * i + c] = (mask && mask[d]) ? 0.0 : p[d];
-            }
+            if (RHS) w[3 * i + c] = (xcur[d] - x0[d]) + kv * v[d];
+            else if (sc) w[3 * i + c] = k > 0 ? z[d] + beta * p[d] : z[d];
+            else w[3 * i + c] = (mask && mask[d]) ? 0.0 : p[d];
+            out[3 * i + c] = 0.0;
         }
     }
-    hex_apply64(X, mat[e], w, RHS ? wm : w, am, ak, lumped, out);
+    // RHS: the mass term, which takes v instead of w, is a pass of its own, needed with Rayleigh mass damping alone
+#pragma unroll 1
+    for (int pass = 0; pass < (RHS && am != 0.0 ? 2 : 1); ++pass) {
+        if (pass == 1)
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int c = 0; c < 3; ++c) w[3 * i + c] = v[3 * (size_t)conn[8 * e + i] + c];
+        hex_apply64(X, mat[e], w, RHS && pass == 0 ? 0.0 : am, pass == 0 ? ak : 0.0, lumped, out);
+    }
     double* st = stage + stage_at(t);
 #pragma unroll
     for (int j = 0; j < 24; ++j) st[64 * j] = out[j];
@@ -277,20 +311,35 @@ __global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slot
                                                          const uint8_t* __restrict__ mask, int pq,
                                                          double* __restrict__ partial, const CgScalars* __restrict__ sc) {
     __shared__ double lds[64];
+    const int first = blockIdx.x * blockDim.x + threadIdx.x;
+    int at[8];  // the node's first staged values, asked for ahead of the scalars
+    auto ask = [&](int i, int b) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            at[u] = i < num_nodes && b + u < slots ? src[(int64_t)(b + u) * num_nodes + i] : -1;
+    };
+    ask(first, 0);
     if (sc && sc->done) return;
     const TV beta = sc && k > 0 ? (TV)(sc->rz[k & 1] / sc->rz[(k - 1) & 1]) : TV(0);
     double acc = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < num_nodes; i += gridDim.x * blockDim.x) {
-        TV s0 = 0, s1 = 0, s2 = 0;
+    for (int i = first; i < num_nodes; i += gridDim.x * blockDim.x) {
+        TV s0 = 0, s1 = 0, s2 = 0, zv[3] = {0, 0, 0}, pv[3] = {0, 0, 0};
+        bool fixed[3] = {false, false, false};
+        if (sc)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int64_t d = 3 * (int64_t)i + c;
+                zv[c] = z[d];
+                pv[c] = p[d];  // not yet written at k == 0, and not used
+                fixed[c] = mask[d];
+            }
         if (y_in) {
             s0 = y_in[3 * (int64_t)i];
             s1 = y_in[3 * (int64_t)i + 1];
             s2 = y_in[3 * (int64_t)i + 2];
         }
         for (int b = 0; b < slots; b += 8) {
-            int at[8];
-#pragma unroll
-            for (int u = 0; u < 8; ++u) at[u] = b + u < slots ? src[(int64_t)(b + u) * num_nodes + i] : -1;
+            if (b > 0 || i != first) ask(i, b);
             TV g[8][3];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
@@ -309,9 +358,9 @@ __global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slot
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const int64_t d = 3 * (int64_t)i + c;
-                const TV pn = k > 0 ? z[d] + beta * p[d] : z[d];
+                const TV pn = k > 0 ? zv[c] + beta * pv[c] : zv[c];
                 p[d] = pn;
-                if (mask[d]) s[c] = pn;
+                if (fixed[c]) s[c] = pn;
                 acc += (double)pn * (double)s[c];
             }
         }
@@ -324,61 +373,19 @@ __global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slot
     }
 }
 
-// FP32 cached operator: stage = A_e p_e of every element, one element per lane, with p = z + beta p_old of CG iteration k
-// formed on the fly (sc null: p as it is). p is zero on BC DOFs without
-// a mask: hex_cg_init_kernel zeroes r there, and the BC rows of the operator are the identity (q = p on them),
-// so r, z and p stay zero on those rows through the solve. The 36 blocks stream in 9 groups of 4 (36 floats =
-// 9 float4 chunks per group). TABLE: A_e is entry table_idx[t] of the distinct-matrix table, staged in LDS by
-// every workgroup (the same floats and the same arithmetic as the per-position cache).
-template <bool TABLE>
-__global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const int* __restrict__ order_pad,
-                                                          const int* __restrict__ conn,
-                                                          const float4* __restrict__ A4,
-                                                          const float4* __restrict__ table,
-                                                          const int* __restrict__ table_idx, int num_distinct,
-                                                          const float* __restrict__ p, float* __restrict__ stage,
-                                                          int k, int max_iter, const float* __restrict__ z,
-                                                          const double* __restrict__ partial, CgScalars* sc) {
-    extern __shared__ float4 lds_table[];
-    __shared__ double lds[64];
-    if (sc && sc->done) return;  // no scalars when the operator is timed alone
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    const int e = t < count_pad ? order_pad[t] : -1;
-    float pv[24], y[24];
-    // the element's inputs are on their way while the block sums of the last iteration are added up
-    if (e >= 0) {
-        const int4* c4 = reinterpret_cast<const int4*>(conn) + 2 * (size_t)e;
-        const int4 n0 = c4[0], n1 = c4[1];
-        const int ids[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
-#pragma unroll
-        for (int a = 0; a < 8; ++a)
-#pragma unroll
-            for (int c = 0; c < 3; ++c) {
-                const int d = 3 * ids[a] + c;
-                if (!sc || k > 0) pv[3 * a + c] = p[d];
-                if (sc) y[3 * a + c] = z[d];
-            }
-    }
-    if (TABLE)
-        for (int i = threadIdx.x; i < num_distinct * kHexChunks; i += blockDim.x) lds_table[i] = table[i];
-    double beta = 0.0;
-    if (sc && !hex_cg_begin(k, max_iter, partial, sc, beta, lds)) return;
-    if (TABLE) __syncthreads();
-    if (e < 0) return;
-#pragma unroll
-    for (int j = 0; j < 24; ++j) {
-        if (sc) pv[j] = k > 0 ? y[j] + (float)beta * pv[j] : y[j];
-        y[j] = 0.f;
-    }
-    const float4* At = A4 + (size_t)(t >> 6) * kHexChunks * 64 + (t & 63);
-    const float4* Tt = TABLE ? lds_table + table_idx[t] * kHexChunks : nullptr;
+// y += A_e p_e from an element's 75 chunks at Ct, one after another (SHARED: in LDS) or 64 apart. The 36 blocks stream in 9
+// groups of 4 (36 floats = 9 float4 chunks per group).
+template <bool SHARED>
+__device__ __forceinline__ void hex_products(const float4* Ct, const float (&pv)[24], float (&y)[24]) {
+    constexpr size_t kStep = SHARED ? 1 : 64;
+    constexpr OffBlocks kOff = off_blocks();
     // the strictly upper blocks, 4 per group of 9 chunks: y_a += B p_b and y_b += B^T p_a
 #pragma unroll
     for (int g = 0; g < 7; ++g) {
         float w[36];
 #pragma unroll
         for (int k = 0; k < 9; ++k) {
-            const float4 v = TABLE ? Tt[9 * g + k] : At[(size_t)(9 * g + k) * 64];
+            const float4 v = Ct[(size_t)(9 * g + k) * kStep];
             w[4 * k] = v.x;
             w[4 * k + 1] = v.y;
             w[4 * k + 2] = v.z;
@@ -386,7 +393,7 @@ __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const i
         }
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-            const int a = off_a(4 * g + m), b = off_b(4 * g + m);
+            const int a = kOff.a[4 * g + m], b = kOff.b[4 * g + m];
             const float* B = w + 9 * m;
 #pragma unroll
             for (int i = 0; i < 3; ++i)
@@ -401,11 +408,8 @@ __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const i
         // two groups (210 registers, 2 waves per SIMD).
         {
             int zero;
-            asm volatile("v_mov_b32 %0, 0" : "=v"(zero) : "v"(y[3 * off_b(4 * g + 3) + 2]));
-            if (TABLE)
-                Tt += zero;
-            else
-                At += zero;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(zero) : "v"(y[3 * kOff.b[4 * g + 3] + 2]));
+            Ct += zero;
         }
     }
     // the diagonal blocks, 4 per group of 6 chunks (symmetric, 6 floats each)
@@ -414,7 +418,7 @@ __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const i
         float w[24];
 #pragma unroll
         for (int k = 0; k < 6; ++k) {
-            const float4 v = TABLE ? Tt[kHexOffFloats / 4 + 6 * g + k] : At[(size_t)(kHexOffFloats / 4 + 6 * g + k) * 64];
+            const float4 v = Ct[(size_t)(kHexOffFloats / 4 + 6 * g + k) * kStep];
             w[4 * k] = v.x;
             w[4 * k + 1] = v.y;
             w[4 * k + 2] = v.z;
@@ -430,6 +434,102 @@ __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const i
             y[3 * a + 2] += B[2] * p0 + B[4] * p1 + B[5] * p2;
         }
     }
+}
+
+// The same products in the same order with one matrix for every lane: its 300 floats lie across the lanes of 5 registers and
+// are read back one by one as scalars (v_readlane). The products then wait for no load; through scalar loads they took 9.5 us
+// at 64x33x65 cubes, each load a wait of its own, with 2 waves on a SIMD to hide it.
+__device__ __forceinline__ void hex_products_scalar(const float (&held)[5], const float (&pv)[24], float (&y)[24]) {
+    auto at = [&](int f) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, held[f >> 6]), f & 63));
+    };
+#pragma unroll
+    for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int b = a + 1; b < 8; ++b) {
+            float B[9];
+#pragma unroll
+            for (int i = 0; i < 9; ++i) B[i] = at(9 * off_index(a, b) + i);
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                y[3 * a + i] += B[3 * i] * pv[3 * b] + B[3 * i + 1] * pv[3 * b + 1] + B[3 * i + 2] * pv[3 * b + 2];
+#pragma unroll
+            for (int j = 0; j < 3; ++j)
+                y[3 * b + j] += B[j] * pv[3 * a] + B[3 + j] * pv[3 * a + 1] + B[6 + j] * pv[3 * a + 2];
+        }
+#pragma unroll
+    for (int a = 0; a < 8; ++a) {
+        float B[6];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) B[i] = at(kHexOffFloats + 6 * a + i);
+        const float p0 = pv[3 * a], p1 = pv[3 * a + 1], p2 = pv[3 * a + 2];
+        y[3 * a] += B[0] * p0 + B[1] * p1 + B[2] * p2;
+        y[3 * a + 1] += B[1] * p0 + B[3] * p1 + B[4] * p2;
+        y[3 * a + 2] += B[2] * p0 + B[4] * p1 + B[5] * p2;
+    }
+}
+
+// FP32 cached operator: stage = A_e p_e of every element, one element per lane, with p = z + beta p_old of CG iteration k
+// formed on the fly (sc null: p as it is). p is zero on BC DOFs without
+// a mask: hex_cg_init_kernel zeroes r there, and the BC rows of the operator are the identity (q = p on them),
+// so r, z and p stay zero on those rows through the solve. kTable: A_e is entry table_idx[t] of the
+// distinct-matrix table, staged in LDS by every workgroup. kOneMatrix: the table has one entry, which comes as scalars:
+// the products read their factors from scalar registers, so that a lane holds 76 vector registers instead of 192 and 6 waves
+// run on a SIMD instead of 2. The same floats and the same arithmetic in every case.
+enum HexSource { kPerPosition, kTable, kOneMatrix };
+template <HexSource SOURCE>
+__global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const int* __restrict__ order_pad,
+                                                          const int* __restrict__ conn,
+                                                          const float4* __restrict__ A4,
+                                                          const float4* __restrict__ table,
+                                                          const int* __restrict__ table_idx, int num_distinct,
+                                                          const float* __restrict__ p, float* __restrict__ stage,
+                                                          int k, int max_iter, const float* __restrict__ z,
+                                                          const double* __restrict__ partial, CgScalars* sc) {
+    extern __shared__ float4 lds_table[];
+    __shared__ double lds[2];
+    // what needs nothing else goes out first: a miss takes near 1 us here, and one load waits for the next
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int e = t < count_pad ? order_pad[t] : -1;
+    HexCgStart start(sc ? k : 0, partial);
+    float held[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
+    if constexpr (SOURCE == kOneMatrix) {
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            const int f = 64 * i + (threadIdx.x & 63);
+            held[i] = reinterpret_cast<const float*>(table)[f < 4 * kHexChunks ? f : 0];
+        }
+    }
+    if (sc && sc->done) return;  // no scalars when the operator is timed alone
+    float pv[24], y[24];
+    // the element's inputs are on their way while the block sums of the last iteration are added up
+    if (e >= 0) {
+        const int4* c4 = reinterpret_cast<const int4*>(conn) + 2 * (size_t)e;
+        const int4 n0 = c4[0], n1 = c4[1];
+        const int ids[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+#pragma unroll
+        for (int a = 0; a < 8; ++a)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int d = 3 * ids[a] + c;
+                if (!sc || k > 0) pv[3 * a + c] = p[d];
+                if (sc) y[3 * a + c] = z[d];
+            }
+    }
+    if (SOURCE == kTable)
+        for (int i = threadIdx.x; i < num_distinct * kHexChunks; i += blockDim.x) lds_table[i] = table[i];
+    double beta = 0.0;
+    if (sc && !start.finish(k, max_iter, sc, beta, lds)) return;
+    if (SOURCE == kTable) __syncthreads();
+    if (e < 0) return;
+#pragma unroll
+    for (int j = 0; j < 24; ++j) {
+        if (sc) pv[j] = k > 0 ? y[j] + (float)beta * pv[j] : y[j];
+        y[j] = 0.f;
+    }
+    if constexpr (SOURCE == kOneMatrix) hex_products_scalar(held, pv, y);
+    else if constexpr (SOURCE == kTable) hex_products<true>(lds_table + table_idx[t] * kHexChunks, pv, y);
+    else hex_products<false>(A4 + (size_t)(t >> 6) * kHexChunks * 64 + (t & 63), pv, y);
     float* st = stage + stage_at(t);
 #pragma unroll
     for (int j = 0; j < 24; ++j) st[64 * j] = y[j];
@@ -1004,15 +1104,14 @@ void elements32(const HexData& h, const float* p, const HexIteration<float>& it,
     const int pad = h.pad_ptr.back();
     const float4* A4 = reinterpret_cast<const float4*>(h.A32);
     if (pad == 0) return;
-    if (h.num_distinct > 0)
-        hipLaunchKernelGGL(hex_apply32_kernel<true>, blocks_for(pad, 256), dim3(256),
-                           (size_t)h.num_distinct * kHexChunks * sizeof(float4), s, pad, h.order_pad, h.conn, A4,
+    auto launch = [&](auto kernel, size_t lds) {
+        hipLaunchKernelGGL(kernel, blocks_for(pad, 256), dim3(256), lds, s, pad, h.order_pad, h.conn, A4,
                            reinterpret_cast<const float4*>(h.table), h.table_idx, h.num_distinct, p, (float*)h.stage,
                            it.k, it.max_iter, it.z, (const double*)it.partial, it.sc);
-    else
-        hipLaunchKernelGGL(hex_apply32_kernel<false>, blocks_for(pad, 256), dim3(256), 0, s, pad, h.order_pad, h.conn, A4,
-                           (const float4*)nullptr, (const int*)nullptr, 0, p, (float*)h.stage, it.k, it.max_iter, it.z,
-                           (const double*)it.partial, it.sc);
+    };
+    if (h.num_distinct == 1) launch(hex_apply32_kernel<kOneMatrix>, 0);
+    else if (h.num_distinct > 1) launch(hex_apply32_kernel<kTable>, (size_t)h.num_distinct * kHexChunks * sizeof(float4));
+    else launch(hex_apply32_kernel<kPerPosition>, 0);
 }
 
 // y = y_in + sign (am M + ak K) w (FP64, matrix-free).
@@ -1222,6 +1321,13 @@ void hex_solve(HexData& h, const HexStepArgs& a, fem_stats& stats, hipStream_t s
             hipLaunchKernelGGL(hex_refine_check_kernel, dim3(1), dim3(kCgThreads), 0, s, a.partial, sweep == 0,
                                o.cg_tolerance, outer, sc);
             if (sweep == o.max_refinements) break;
+            // a sweep beyond those of the last step is looked at before its iterations are queued
+            const bool look = sweep >= h.predicted_sweeps && sweep > 0;
+            if (look) {
+                HCHECK(hipMemcpyAsync(a.h_sc + 1, outer, sizeof(CgScalars), hipMemcpyDeviceToHost, s));
+                HCHECK(hipStreamSynchronize(s));
+                if (a.h_sc[1].done) break;
+            }
             hipLaunchKernelGGL((hex_cg_init_kernel<float>), dim3(kCgBlocks), dim3(kCgThreads), 0, s, n, a.r64,
                                diag32, (float*)a.vec[0], (float*)a.vec[1], (float*)a.vec[2], (float*)a.vec[5],
                                a.bcmask, a.partial, (const CgScalars*)outer);
@@ -1230,14 +1336,17 @@ void hex_solve(HexData& h, const HexStepArgs& a, fem_stats& stats, hipStream_t s
             const int it = run_hex_cg<float>(h, a, true, sc, a.h_sc, a.predicted[ps], (float*)a.vec[0],
                                              (float*)a.vec[1], (float*)a.vec[2], (float*)a.vec[3], (float*)a.vec[4],
                                              (float*)a.vec[5], s);
-            HCHECK(hipMemcpyAsync(a.h_sc + 1, outer, sizeof(CgScalars), hipMemcpyDeviceToHost, s));
-            HCHECK(hipStreamSynchronize(s));
-            if (a.h_sc[1].done) break;
+            if (!look) {
+                HCHECK(hipMemcpyAsync(a.h_sc + 1, outer, sizeof(CgScalars), hipMemcpyDeviceToHost, s));
+                HCHECK(hipStreamSynchronize(s));
+                if (a.h_sc[1].done) break;
+            }
             total += it + 1;
             hipLaunchKernelGGL(hex_accumulate_kernel, dim3(kCgBlocks), dim3(kCgThreads), 0, s, n,
                                (const float*)a.vec[0], a.dv, outer);
             sweeps++;
         }
+        h.predicted_sweeps = sweeps;
         CgScalars oh;
         HCHECK(hipMemcpyAsync(&oh, outer, sizeof(CgScalars), hipMemcpyDeviceToHost, s));
         HCHECK(hipStreamSynchronize(s));

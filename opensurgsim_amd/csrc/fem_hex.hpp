@@ -47,6 +47,7 @@ struct HexData {
     float* diagx32 = nullptr;
     double a32_cm = 0.0, a32_ck = 0.0;  // coefficients of M and K the cached A32 / diagonal were built for
     int a32_lumped = -1;                // lumped mass flag of the cache (-1: not built)
+    int predicted_sweeps = 0;           // refinement sweeps of the last solve
     bool ready = false;
 };
 
