@@ -184,3 +184,44 @@ def test_direct_solver_rejections():
         g.set_instances(b.node_offsets, b.dt)
     assert e.value.code == femgpu.FEM_ERR_INVALID
     g.close()
+
+
+# bandwidths 20, then 128, 134, 254, 257, 380, 386, 512 and 515 (the one-column solve's variants and its limit), 1,022 and 1,025; DOF counts with remainders of 32-column panels and 64-row blocks
+@pytest.mark.parametrize("n", [(1, 1, 1), (6, 5, 5), (7, 9, 3), (5, 10, 6), (6, 3, 16),
+                               (2, 7, 13), (2, 6, 15), (2, 8, 16), (2, 7, 18), (1, 15, 19), (1, 9, 30)])
+def test_lu_factor_and_solve_over_bandwidths(n):
+    """A column solved by itself, 3, 63, 64 and 65 at once (past 64 in two parts) against the dense inverse of the oracle:
+    1e-12 of the largest entry, as for the other compliance tests at these sizes."""
+    cfg = mg.config_linear_cpu(n)
+    o = make_oracle(cfg, scheme=oracle.LINEAR_EULER_IMPLICIT, linsolver=oracle.LU)
+    o.set_compliance_at_first_linear_step(True)
+    o.step(cfg.dt, 1)
+    C = o.compliance_matrix()
+    g = make_gpu(cfg, scheme=femgpu.EULER_IMPLICIT, linear_solver=femgpu.LINEAR_SOLVER_LU)
+    assert g.step(1) == femgpu.FEM_OK
+    conn = np.asarray(cfg.conn)
+    say("%d DOF, nodes of an element up to %d apart" % (cfg.x0.size, (conn.max(axis=1) - conn.min(axis=1)).max()))
+    B = np.random.default_rng(11).normal(size=(cfg.x0.size, 65))
+    Xr = C @ B
+    for m in (1, 3, 63, 64, 65):
+        X = g.apply_compliance(B[:, :m])
+        err = np.abs(X.reshape(cfg.x0.size, m) - Xr[:, :m]).max() / np.abs(Xr).max()
+        say("  %d columns: %.2e" % (m, err))
+        assert err <= 1e-12
+    g.close()
+
+
+@pytest.mark.parametrize("n", [(119, 6, 6), (121, 6, 6), (122, 6, 6)])
+def test_lu_column_solve_at_its_largest(n):
+    """17,640 and 17,934 DOFs, where a column fills the local memory, and 18,081, past the limit, against conjugate gradients
+    on the same operator at 1e-14: 1e-9 of the norm, as the condition of the bar is below 1e5."""
+    cfg = mg.config_linear_cpu(n)
+    g = make_gpu(cfg, linear_solver=femgpu.LINEAR_SOLVER_LU)
+    r = make_gpu(cfg, tol=1e-14)
+    assert g.step(1) == femgpu.FEM_OK and r.step(1) == femgpu.FEM_OK
+    B = np.random.default_rng(12).normal(size=(cfg.x0.size, 2))
+    err = rel(g.apply_compliance(B), r.apply_compliance(B))
+    say("%d DOF: %.2e" % (cfg.x0.size, err))
+    assert np.isfinite(err) and err <= 1e-9
+    g.close()
+    r.close()
