@@ -95,8 +95,10 @@ FUSED_SUMS, CG_BLOCKS = 7, 512
 
 
 def cg_kernel_name(w):
-    """The dominant kernel of the CG iteration: the library runs one fused kernel per iteration unless
-    FEM_CG_KERNELS=split selects the operator + vector kernel pair (its operator kernel is then timed)."""
+    """The kernel of one CG iteration that streams the operator: the fused kernel, or with FEM_CG_KERNELS=split the
+    operator kernel of the operator + vector pair. Steps whose operator fits the chip's registers run a whole solve
+    in one launch instead (cg_resident_kernel), which reads the operator from HBM once per solve and has no HBM
+    roofline per iteration; FEM_CG_KERNELS=fused keeps the launch per iteration."""
     t = "float" if w == 4 else "double"
     split = os.environ.get("FEM_CG_KERNELS", "") == "split"
     return ("cg_apply_kernel<%s>" if split else "cg_fused_kernel<%s>") % t
@@ -268,12 +270,11 @@ def bench_hex(args):
                     v=float(np.linalg.norm(r["v"] - r64["v"]) / np.linalg.norm(r64["v"])))
     e32, et = err(r32), err(rt)
     log("fp32+refine vs fp64 rel err", e32, "table", et, "identical", bool(np.array_equal(r32["x"], rt["x"])))
-    # one application of the FP32 operator (8 colours on a block mesh): per element the cached packed upper
-    # triangle (300 floats, 1,200 B; table: a 4 B index), 32 B of node ids and its 4 B slot; per colour p read
-    # and q read and written over the DOFs
-    colours = 8
-    cache_bytes = E * (1200 + 32 + 4) + colours * 12 * D
-    table_bytes = E * (4 + 32 + 4) + colours * 12 * D
+    # one application of the FP32 operator: per element the cached packed upper triangle (300 floats, 1,200 B; table:
+    # a 4 B index), 32 B of node ids and its 4 B slot; p read and q written over the DOFs. The products staged between
+    # the two kernels (96 B written and read per element) are not counted
+    cache_bytes = E * (1200 + 32 + 4) + 8 * D
+    table_bytes = E * (4 + 32 + 4) + 8 * D
     return {"metric": METRIC, "value": D * steps / r32["seconds"], "unit": "DOF-steps/s", "n_gpus": 1,
             "steps": steps, "warmup": args.warmup, "ms_per_step": 1e3 * r32["seconds"] / steps,
             "higher_is_better": True, "scaling": "weak", "vs_baseline": None, "dtype": "f32+f64refine",
@@ -282,12 +283,12 @@ def bench_hex(args):
                                    "element + FP64 refinement 1e-6, dt=1ms" % n, "elements": int(E), "nodes": int(N),
                        "dof": int(D), "parallelism": "single-gpu"},
             "rel_err_vs_fp64": e32,
-            "roofline": roofline("hex_apply32_kernel<false> (all 8 colours)", cache_bytes, r32["op_ms"] / 1e3),
+            "roofline": roofline("hex_apply32_kernel + hex_gather_kernel (a matrix per element)", cache_bytes, r32["op_ms"] / 1e3),
             "table_variant": {"value": D * steps / rt["seconds"], "ms_per_step": 1e3 * rt["seconds"] / steps,
                               "distinct_element_matrices": rt["distinct"], "rel_err_vs_fp64": et,
                               "identical_to_per_element_cache": bool(np.array_equal(r32["x"], rt["x"]) and
                                                                      np.array_equal(r32["v"], rt["v"])),
-                              "roofline": roofline("hex_apply32_kernel<true> (all 8 colours)", table_bytes,
+                              "roofline": roofline("hex_apply32_kernel + hex_gather_kernel (distinct matrices)", table_bytes,
                                                    rt["op_ms"] / 1e3)},
             "fp64": {"value": D * steps / r64["seconds"], "ms_per_step": 1e3 * r64["seconds"] / steps,
                      "cg_iters_per_step": r64["cg"] / steps, "operator_ms": r64["op_ms"]},
@@ -511,7 +512,8 @@ def bench_adjoint(args):
     N = cfg.x0.shape[0]
     Bk = g.num_nonzeros() // 9
     roof = roofline("cg_fused_kernel<double>", spmv_bytes((N, 3 * N, Bk), 8), op_ms / 1e3,
-                    "the forward and transpose solves' CG iteration; operator and vectors (11.5 MB) stay in the MALL")
+                    "the launch-per-iteration form of the solves' CG iteration; the solves themselves hold the operator "
+                    "in registers (cg_resident_kernel, one launch each)")
     out = {"metric": METRIC, "value": reps / t, "unit": "gradients/s", "n_gpus": 1, "steps": reps,
            "roofline": roof,
            "warmup": 1, "ms_per_step": 1e3 * t / reps, "higher_is_better": True, "scaling": "weak",
@@ -740,6 +742,9 @@ def bench_corotational(args):
         "roofline": {"bound": "hbm", "kernel": cg_kernel_name(w), "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
                      "algorithmic_bytes_per_launch": bytes_per, "avg_launch_us": sp_avg_s * 1e6,
+                     "note": "the kernel of the launch-per-iteration path, timed by itself; a step's solve launches "
+                             "(in_step_launches, avg_launch_us_in_step_events) are whole inner solves with the "
+                             "operator in registers unless FEM_CG_KERNELS=fused or split",
                      "avg_launch_us_in_step_events": 1e3 * sp_ms / max(sp_n, 1), "in_step_launches": sp_n,
                      "measured_copy_GBps": copy_gbs},
         "cpu_baseline": cpu,

@@ -171,15 +171,16 @@ int fem_set_state(fem_ctx* ctx, const double* x, const double* v);
  * the first step. The step statistics are left as the last step set them. */
 int fem_apply_compliance(fem_ctx* ctx, const double* b, int64_t num_columns, double* out);
 /* The same with device pointers (column-major, ndof x num_columns), ordered on the context stream. On a
- * tetrahedral mesh the columns are solved up to 8 at a time by a multi-column FP64 CG that reads the
- * operator once per iteration for all of them (each column keeps its own Eigen CG recurrence and test). */
+ * tetrahedral mesh each column keeps its own Eigen CG recurrence and test in FP64. Where the operator fits the
+ * chip's registers the columns run side by side in launches that hold it there; otherwise (and where b and out
+ * overlap) up to 8 at a time by a multi-column CG that reads the operator once per iteration for all of them. */
 int fem_apply_compliance_device(fem_ctx* ctx, const double* b, int64_t num_columns, double* out);
 /* The same as fem_apply_compliance_device, allocating nothing: no hipMalloc, hipFree, hipHostMalloc or other
  * allocating routine. No counterpart in the reference; it is for callers that cannot allocate (code under HIP
- * graph capture, tight serving loops, harnesses that forbid allocation). The multi-column CG works in a fixed
+ * graph capture, tight serving loops, harnesses that forbid allocation). The solves work in a fixed
  * device workspace of FEM_NOALLOC_SCRATCH_BYTES per GPU, held from fem_create until the process ends, which
  * bounds the mesh to about 256,000 DOFs (larger meshes: FEM_ERR_INVALID with the limit in the message). Every
- * column goes through the multi-column FP64 CG (in FP64 mode the results equal fem_apply_compliance_device's
+ * column goes through an FP64 CG (in FP64 mode the results equal fem_apply_compliance_device's
  * bit for bit; in the FP32 + refinement mode they agree to the CG tolerance). Tetrahedral meshes of one
  * instance only; FEM_ERR_ORDER before the first step and after boundary conditions were added since the last
  * step. All contexts on one GPU share its workspace and each call leaves its contents behind: calls that
@@ -204,7 +205,7 @@ int fem_get_compliance_matrix_device(fem_ctx* ctx, double* out);  /* device outp
  * per node; scale: the builder's dt * scale; fixed point: the three unit axes, frictionless contact: the
  * normal). cht (host, ndof x num_directions column-major, or NULL) = C H^T with C applied as
  * fem_apply_compliance does; hcht (host, num_directions^2 row-major, or NULL) = H C H^T. The H^T columns are
- * built and solved on the device (multi-column CG on tetrahedral meshes). FEM_ERR_ORDER before the first step. */
+ * built and solved on the device (fem_apply_compliance_device on tetrahedral meshes). FEM_ERR_ORDER before the first step. */
 int fem_constraint_compliance(fem_ctx* ctx, int64_t element, const double* coordinate, int num_directions,
                               const double* directions, double scale, double* cht, double* hcht);
 int fem_get_state(fem_ctx* ctx, double* x, double* v);

@@ -2579,7 +2579,7 @@ void compliance_lu(fem_ctx* c, const double* b, int64_t ncols, double* out, doub
         const int cnt = (int)std::min<int64_t>(tmp_cols, ncols - j0);
         for (int j = 0; j < cnt; ++j)
             launch_masked_copy(n, b + (size_t)(j0 + j) * n, c->bcmask.p, tmp + (size_t)j * n, c->stream);
-        launch_band_solve(c->lu, cnt, tmp, n, out + (size_t)j0 * n, n, c->stream);
+        launch_band_solve(c->lu, cnt, tmp, n, out + (size_t)j0 * n, n, c->stream, -1, ncols);
         launch_zero_masked_rows(n, cnt, c->bcmask.p, out + (size_t)j0 * n, c->stream);
     }
 }

@@ -34,16 +34,16 @@ size_t band_bytes(int64_t n, int bw);
 // blk_row[k], block column colidx[k]) scattered into band storage of bandwidth bw (zero elsewhere).
 void launch_band_fill(DeviceBandLU& lu, int64_t num_blocks, const int* blk_row, const int* colidx, const double* S,
                       hipStream_t s);
-// In-place factorization of the band storage (the lower triangle is read): panels of 32 columns, each the
-// panel's rows eliminated against its diagonal block and the rank-32 update of the trailing bw x bw lower
-// triangle by LDS-tiled workgroups; then the inverses of the diagonal blocks.
+// In-place factorization of the band storage (the lower triangle is read): panels of 32 columns, each one launch of
+// LDS-tiled workgroups over the trailing bw x bw lower triangle; then L and the inverses of the diagonal blocks.
 void launch_band_factor(DeviceBandLU& lu, hipStream_t s);
 // x = A^-1 b for nrhs columns (column j at b + j * ldb and x + j * ldx; x may alias b): forward substitution
-// with L and back substitution with U by 64-row blocks, one workgroup per 16 columns (4 below 64 columns).
+// with L and back substitution with U by 64-row blocks, one workgroup per column (up to 256 columns of a request, narrow
+// bands) or per 16 columns (4 below 64 columns). total: columns of the request that nrhs is a part of.
 // identity_first >= 0: b holds columns identity_first .. of the identity, and the forward pass skips the rows
 // above each workgroup's first column (their solutions are zero).
 void launch_band_solve(const DeviceBandLU& lu, int nrhs, const double* b, int64_t ldb, double* x, int64_t ldx,
-                       hipStream_t s, int64_t identity_first = -1);
+                       hipStream_t s, int64_t identity_first = -1, int64_t total = 0);
 // Columns [first, first + count) of the identity (n rows each, column-major with leading dimension n).
 void launch_identity_columns(int64_t n, int64_t first, int count, double* out, hipStream_t s);
 // Rows and columns of the boundary DOFs (mask != 0) of an n x count column block (columns first.. of an n x n

@@ -108,3 +108,47 @@ def test_hex_distinct_matrix_table(monkeypatch):
     say("  perturbed mesh: distinct", g.hex_distinct_matrices(), "errors", e)
     assert g.hex_distinct_matrices() == 0
     assert e["u"] < 1e-6 and e["v"] < 1e-6
+
+
+@pytest.mark.parametrize("moduli", [1, 2, 32, 33])
+def test_hex_operator_by_number_of_matrices(moduli, monkeypatch):
+    """One distinct matrix (kept in registers), a few (the table, to its limit of 32) and more (one per element) on an odd-sized
+    block of 525 elements, which ends in a part-filled tile: the same floats in the same order, so the trajectory is that of the
+    per-element cache bit for bit."""
+    cfg = mg.config_hex((7, 5, 15))
+    # a block's cubes repeat to the last bit only where their node coordinates do: snap the edge to a power of two
+    cfg["x0"] = np.round(cfg.x0 / cfg.h) / 64.0
+    cfg["E"] = 2e4 * (1.0 + (np.arange(cfg.conn.shape[0]) * 7 % moduli) / 64.0)
+    runs = []
+    for flag in ("1", "0"):
+        monkeypatch.setenv("FEM_HEX_TABLE", flag)
+        g = make_gpu(cfg, precision=femgpu.FP32_REFINED, tol=1e-9)
+        assert g.step(3) == femgpu.FEM_OK
+        runs.append((g.state(), g.hex_distinct_matrices(), g.stats()["total_cg_iterations"]))
+        g.close()
+    say("moduli", moduli, "distinct", runs[0][1], "iterations", runs[0][2])
+    assert runs[0][1] == (moduli if moduli <= 32 else 0) and runs[1][1] == 0
+    assert np.array_equal(runs[0][0][0], runs[1][0][0]) and np.array_equal(runs[0][0][1], runs[1][0][1])
+    assert runs[0][2] == runs[1][2]
+
+
+@pytest.mark.parametrize("precision,bound", [(femgpu.FP64, 1e-9), (femgpu.FP32_REFINED, 1e-6)])
+@pytest.mark.parametrize("spokes", [3, 6, 9])
+def test_hex_nodes_of_many_elements(spokes, precision, bound):
+    """Hexahedra around an axis, two layers: the middle node belongs to 6, 12 and 18 elements (8 on a block), each in a colour of its
+    own; the trajectory within the bounds of the block's."""
+    cfg = mg.config_hex((2, 2, 2))
+    ring = 2 * spokes
+    a = 2 * np.pi * np.arange(ring) / ring
+    rad = 0.01 * np.where(np.arange(ring) % 2, 1.3, 1.0)
+    layer = np.vstack([[0.0, 0.0], np.stack([rad * np.cos(a), rad * np.sin(a)], 1)])
+    N = ring + 1
+    x0 = np.vstack([np.column_stack([layer, np.full(N, 0.01 * k)]) for k in range(3)])
+    quads = np.array([[0, 1 + 2 * i, 2 + 2 * i, 1 + (2 * i + 2) % ring] for i in range(spokes)])
+    conn = np.vstack([np.hstack([quads + k * N, quads + (k + 1) * N]) for k in range(2)]).astype(cfg.conn.dtype)
+    ne = conn.shape[0]
+    cfg.update(x0=x0, conn=conn, E=np.full(ne, 2e4), nu=np.full(ne, 0.45), rho=np.full(ne, 1050.0),
+               bc_nodes=np.arange(N, dtype=cfg.bc_nodes.dtype), v0=np.zeros(x0.size), fext=None)
+    e = trajectory(cfg, 5, precision, 1e-12, 1e-12 if precision == femgpu.FP64 else 1e-9)
+    say("spokes", spokes, "precision", precision, e)
+    assert e["u"] < bound and e["v"] < bound
