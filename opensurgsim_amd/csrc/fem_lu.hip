@@ -711,11 +711,11 @@ void launch_band_solve(const DeviceBandLU& lu, int nrhs, const double* b, int64_
                        hipStream_t s, int64_t identity_first, int64_t total) {
     if (nrhs <= 0 || lu.n == 0) return;
     // A workgroup per column: 1 column 0.32 ms against 1.43 with the tiled kernel at 3,240 DOFs, bandwidth 356; 64 columns
-    // 0.52 against 2.53 (0.26 and 0.57 at 1,488 x 77, 0.88 and 4.9 at 5,184 x 470), 256 in four parts 1.9. Past 256 the tiled
-    // kernel's one launch for all of them is as fast or faster. The line is drawn by the whole request (total), so that
-    // its results do not depend on how a caller cuts it. Columns of the identity stay with the tiled kernel, which skips
-    // the rows above them.
-    if (std::max<int64_t>(nrhs, total) <= 256 && identity_first < 0 && lu.bw <= kColumnMaxBw && lu.n <= kColumnMaxN) {
+    // 0.52 against 2.53 (0.26 and 0.57 at 1,488 x 77, 0.88 and 4.9 at 5,184 x 470); 512 in one launch 1.9 against 4.1 (1.3 and
+    // 2.3, 2.5 and 6.4). Two more rounds of 256 workgroups would bring the two level near 1,000. The line is drawn by the
+    // whole request (total), so that its results do not depend on how a caller cuts it. Columns of the identity stay with
+    // the tiled kernel, which skips the rows above them.
+    if (std::max<int64_t>(nrhs, total) <= 512 && identity_first < 0 && lu.bw <= kColumnMaxBw && lu.n <= kColumnMaxN) {
         if (lu.bw <= 128) return solve_columns<2>(lu, nrhs, b, ldb, x, ldx, s);
         if (lu.bw <= 256) return solve_columns<4>(lu, nrhs, b, ldb, x, ldx, s);
         if (lu.bw <= 384) return solve_columns<6>(lu, nrhs, b, ldb, x, ldx, s);

@@ -38,7 +38,7 @@ void launch_band_fill(DeviceBandLU& lu, int64_t num_blocks, const int* blk_row, 
 // LDS-tiled workgroups over the trailing bw x bw lower triangle; then L and the inverses of the diagonal blocks.
 void launch_band_factor(DeviceBandLU& lu, hipStream_t s);
 // x = A^-1 b for nrhs columns (column j at b + j * ldb and x + j * ldx; x may alias b): forward substitution
-// with L and back substitution with U by 64-row blocks, one workgroup per column (up to 256 columns of a request, narrow
+// with L and back substitution with U by 64-row blocks, one workgroup per column (up to 512 columns of a request, narrow
 // bands) or per 16 columns (4 below 64 columns). total: columns of the request that nrhs is a part of.
 // identity_first >= 0: b holds columns identity_first .. of the identity, and the forward pass skips the rows
 // above each workgroup's first column (their solutions are zero).

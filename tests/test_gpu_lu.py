@@ -186,11 +186,12 @@ def test_direct_solver_rejections():
     g.close()
 
 
-# bandwidths 20, then 128, 134, 254, 257, 380, 386, 512 and 515 (the one-column solve's variants and its limit), 1,022 and 1,025; DOF counts with remainders of 32-column panels and 64-row blocks
+# bandwidths 20, then 128, 134, 254, 257, 380, 386, 512 and 515 (the one-column solve's variants and its limit), 1,022 and
+# 1,025; DOF counts with remainders of 32-column panels and 64-row blocks
 @pytest.mark.parametrize("n", [(1, 1, 1), (6, 5, 5), (7, 9, 3), (5, 10, 6), (6, 3, 16),
                                (2, 7, 13), (2, 6, 15), (2, 8, 16), (2, 7, 18), (1, 15, 19), (1, 9, 30)])
 def test_lu_factor_and_solve_over_bandwidths(n):
-    """A column by itself, 3 to 65 (past 64 in parts), 256 and 257 (the tiled solve) against the dense inverse of the oracle:
+    """A column by itself, 3 to 65 (past 64 in parts), 512 and 513 (the tiled solve) against the dense inverse of the oracle:
     1e-12 of the largest entry, as for the other compliance tests at these sizes."""
     cfg = mg.config_linear_cpu(n)
     o = make_oracle(cfg, scheme=oracle.LINEAR_EULER_IMPLICIT, linsolver=oracle.LU)
@@ -201,9 +202,9 @@ def test_lu_factor_and_solve_over_bandwidths(n):
     assert g.step(1) == femgpu.FEM_OK
     conn = np.asarray(cfg.conn)
     say("%d DOF, nodes of an element up to %d apart" % (cfg.x0.size, (conn.max(axis=1) - conn.min(axis=1)).max()))
-    B = np.random.default_rng(11).normal(size=(cfg.x0.size, 257))
+    B = np.random.default_rng(11).normal(size=(cfg.x0.size, 513))
     Xr = C @ B
-    for m in (1, 3, 63, 64, 65, 256, 257):
+    for m in (1, 3, 63, 64, 65, 512, 513):
         X = g.apply_compliance(B[:, :m])
         err = np.abs(X.reshape(cfg.x0.size, m) - Xr[:, :m]).max() / np.abs(Xr).max()
         say("  %d columns: %.2e" % (m, err))
