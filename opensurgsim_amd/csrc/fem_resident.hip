@@ -250,8 +250,10 @@ __global__ __launch_bounds__(kResThreads, 2) void cg_resident_kernel(ResidentArg
         const int cnt = a.t.lane_info[li] & 0xff;
         pi = 3 * (a.t.lane_info[li] >> 8);
         const TV* S = (const TV*)a.S + 9 * (int64_t)a.t.lane_k0[li];
+        // every lane loads nb blocks (its last one again, the operator's first one where it has none), so that no load waits on
+        // a branch
 #pragma unroll
-        for (int s = 0; s < NB; ++s) {  // every lane loads nb blocks (its last one again), so that no load waits on a branch
+        for (int s = 0; s < NB; ++s) {
             const TV* B = S + 9 * (s < cnt ? s : max(cnt - 1, 0));
 #pragma unroll
             for (int i = 0; i < 9; ++i) m[s][i] = B[i];
@@ -700,7 +702,9 @@ bool plan_group(ResidentPlan& plan, int g, int64_t i0, int64_t i1, int64_t n0, c
                 continue;
             }
             const Share& sh = shares[lane];
-            plan.lane_k0[li] = sh.k0;
+            // a row without blocks (a node in no element) starts at 0: the kernel loads a first block all the same, and its
+            // own place is past the operator's end where no later row has blocks
+            plan.lane_k0[li] = sh.cnt > 0 ? sh.k0 : 0;
             plan.lane_info[li] = sh.cnt | sh.part << 8;
             for (int s = 0; s < sh.cnt; ++s)
                 plan.cols[((size_t)g * nb + s) * kResThreads + lane] = (uint16_t)local[ci[sh.k0 + s]];
