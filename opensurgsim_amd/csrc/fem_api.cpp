@@ -16,6 +16,7 @@
 #include "fem_lu.hpp"
 #include "fem_mcg.hpp"
 #include "fem_resident.hpp"
+#include "fem_share.hpp"
 
 #include <hip/hip_runtime.h>
 
@@ -26,7 +27,6 @@
 #include <cstring>
 #include <limits>
 #include <map>
-#include <mutex>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -557,11 +557,13 @@ bool use_resident(const fem_ctx* c, bool fp32) {
 
 constexpr int kResBackoff = 256;  // solves with one launch per iteration after a one-launch solve gave up
 
-// One-launch solves of a device go one after another: two of them side by side could each hold CUs that the other's
-// workgroups wait for. Held from the launch until the host has seen the solve's end.
-std::mutex& resident_mutex(int device) {
-    static std::mutex mu[64];
-    return mu[(unsigned)device % 64];
+// One-launch solves of the contexts of a device share its CUs. Held from the launch until the host has seen the solve's end,
+// for the largest launch of the solve. A frame of a 7x8x6 block beside the 250 iterations of a stiff 14^3 block takes 0.16 ms, as
+// alone; one lock for all solves made it 1.00 ms, and a launch per iteration for both 0.39. Eight stiff 14^3 blocks on threads of
+// their own: 2,261 frames a second, 867 with one lock, 591 with a launch per iteration.
+ChipShare::Use share_chip(const fem_ctx* c, int workgroups) {
+    static ChipShare chips[64];
+    return ChipShare::Use(chips[(unsigned)c->device % 64], workgroups, c->num_cus);
 }
 
 ResidentArgs resident_args(fem_ctx* c) {
@@ -661,7 +663,7 @@ int64_t max_iters(fem_ctx* c) {
 int run_cg_iterations(fem_ctx* c, const CgArgs& a, const double* b, int max_iter) {
     int& pred = c->solving_adjoint ? c->predicted_adj : c->predicted_iters;
     if (a.slots) {
-        std::lock_guard<std::mutex> one(resident_mutex(c->device));
+        const ChipShare::Use cus = share_chip(c, c->res.groups);
         TIMED(c, FEM_PHASE_SPMV, 0, launch_resident(c, a, max_iter));
         HIPCHECK(hipMemcpyAsync(c->h_sc, a.sc, sizeof(CgScalars), hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(hipStreamSynchronize(c->stream));
@@ -783,8 +785,8 @@ void linear_solve(fem_ctx* c) {
     CgArgs a = cg_args(c, true, c->opt.inner_tolerance);
     a.floor_tol = kInnerFloor * c->opt.cg_tolerance;
     if (max_iter < 1) a.slots = nullptr;
-    std::unique_lock<std::mutex> one(resident_mutex(c->device), std::defer_lock);
-    if (a.slots) one.lock();
+    ChipShare::Use cus;
+    if (a.slots) cus = share_chip(c, c->res.groups);
     CgScalars* outer = c->scal.p + 1;
     // One-kernel CG path: sweep s is one launch for dv_s = dv_{s-1} + x_{s-1}, the FP64 residual and the inner
     // solve's start, and one for the outer test with the inner scalars; dv_s and x_s alternate between two
@@ -857,7 +859,7 @@ void linear_solve(fem_ctx* c) {
         // an inner solve gave up waiting for a workgroup: the solve starts over with one launch per iteration
         c->res_backoff = kResBackoff;
         c->res_dirty = true;
-        one.unlock();
+        cus.release();
         return linear_solve(c);
     }
     // sweeps that applied a correction recorded their inner iteration counts
@@ -1355,7 +1357,7 @@ int run_batch_solves(fem_ctx* c, const BatchCg& a, const double* b, const CgScal
     const int M = c->num_instances;
     bool gave_up = false, rest = false;
     {
-        std::lock_guard<std::mutex> one(resident_mutex(c->device));
+        const ChipShare::Use cus = share_chip(c, *std::max_element(c->res_launches.begin(), c->res_launches.end()));
         ResidentArgs r = resident_args(c);
         r.S = a.S;
         r.r = a.r;
@@ -2532,7 +2534,7 @@ ColumnWork column_work(double* base, CgScalars* sc, size_t n, int columns) {
 bool resident_columns(fem_ctx* c, const double* b, int64_t ncols, double* out, const ColumnWork& w) {
     const size_t n = (size_t)c->ndof;
     CgScalars h[kResColumnStates];
-    std::lock_guard<std::mutex> one(resident_mutex(c->device));
+    const ChipShare::Use cus = share_chip(c, c->res.groups * (int)std::min<int64_t>(c->res_columns, ncols));
     for (int64_t j0 = 0; j0 < ncols; j0 += kResColumnStates) {
         const int some = (int)std::min<int64_t>(kResColumnStates, ncols - j0);
         for (int j = 0; j < some; j += c->res_columns) {

@@ -8,6 +8,7 @@ follow their own rounding, so their counts are not compared.
 """
 import functools
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -154,6 +155,46 @@ def test_repeats_bit_for_bit_and_from_threads(monkeypatch):
         t.join(60)
     for w, g in zip(want, got):
         assert np.array_equal(w[0], g[0]) and np.array_equal(w[1], g[1])
+
+
+def test_small_body_beside_a_long_solve():
+    """A body of 4 workgroups steps beside one of 25 whose solves take hundreds of iterations, on its own stream from another
+    thread: it does not wait for the other's solve to end. Its median frame is held to half of the other's; it took 0.16 of it
+    alone and all of it when one solve kept out every other one."""
+    def body(n, young):
+        x0, tets, bc = block(n)
+        g = femgpu.FemGpu(0)
+        g.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets, young, 0.45, 1000.0)
+        g.add_bc_nodes(bc)
+        g.set_options(dt=1e-3, cg_tolerance=1e-8)
+        return g, x0, 0.01 * np.random.RandomState(1).standard_normal(x0.size)
+
+    def frames(b, more):
+        t, i = [], 0
+        while more(i):
+            if i % 10 == 0:
+                b[0].set_state(b[1], b[2])
+            t0 = time.perf_counter()
+            assert b[0].step(1) == femgpu.FEM_OK
+            t.append(time.perf_counter() - t0)
+            i += 1
+        return sorted(t)[len(t) // 2]
+
+    small, large = body((7, 8, 6), 5e4), body((14, 14, 14), 5e6)
+    for b in (small, large):
+        frames(b, lambda i: i < 20)
+    stop, got = threading.Event(), []
+    thread = threading.Thread(target=lambda: got.append(frames(large, lambda i: not stop.is_set())))
+    thread.start()
+    try:
+        beside = frames(small, lambda i: i < 300)
+    finally:
+        stop.set()
+        thread.join(60)
+    print("median frame beside: %.3f ms, the other's %.3f ms" % (1e3 * beside, 1e3 * got[0]), flush=True)
+    assert beside < 0.5 * got[0]
+    small[0].close()
+    large[0].close()
 
 
 def run_batch(sizes, precision, steps=2):
