@@ -188,6 +188,19 @@ struct PhaseTimer {
 
 }  // namespace
 
+// One-launch CG solves of a context in one precision (fem_resident.hip): the partition, exchanged vectors, published sums. Each
+// precision keeps its own: a program that changes between them would wait for the host's partition each time (3 ms at 40^3).
+struct Resident {
+    bool planned = false;             // for this mesh and these instances; t.groups == 0: the operator does not fit the chip
+    ResidentTables t;
+    std::vector<int> launches;        // batch: workgroups of each launch
+    std::vector<uint8_t> instances;   // batch: the instances these solve
+    int columns = 1;                  // columns that fit one launch
+    bool dirty = false;               // the exchanged vectors have to be emptied (new, or left by a solve that gave up)
+    DevBuf<unsigned char> mem, exch;
+    DevBuf<unsigned long long> slots;
+};
+
 struct fem_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -240,19 +253,11 @@ struct fem_ctx {
     DevBuf<unsigned char> cg_x2;  // FP32 refinement: inner solution of the odd sweeps
     DevBuf<unsigned char> cg_r1, cg_z1, cg_q1, cg_w0, cg_w1;                    // fused CG: second buffers
     DevBuf<double> part7;      // [2][kFusedSums * kCgBlocks] block sums of the fused CG kernel, by parity
-    // one-launch CG solves (fem_resident.hip): the partition for res_precision, exchanged vectors, published sums
-    ResidentTables res;
-    std::vector<int> res_launches;        // batch: workgroups of each launch
-    std::vector<uint8_t> res_instances;   // batch: the instances these solve
-    int res_columns = 1;                  // columns that fit one launch
-    DevBuf<double> res_col;               // their r, z, preconditioner and partial sums
+    Resident res[2];           // one-launch CG solves in FP64 and FP32
+    DevBuf<double> res_col;    // compliance columns: their r, z, preconditioner and partial sums
     DevBuf<CgScalars> res_col_sc;
-    int res_precision = -1;
     std::vector<double> h_x0;  // rest positions, for the partition
-    bool res_dirty = false;    // the exchanged vectors have to be emptied (new, or left by a solve that gave up)
     int res_backoff = 0;       // solves left to run with one launch per iteration after one gave up
-    DevBuf<unsigned char> res_mem, res_exch;
-    DevBuf<unsigned long long> res_slots;
     int num_cus = 0;
     long long res_wait_ticks = 400000;  // 4 ms; FEM_CG_WAIT_US
     DevBuf<double> partial;    // [4 * kCgBlocks] block sums of the grid reductions
@@ -497,10 +502,11 @@ Operator op_of(fem_ctx* c) {
 // The partition of a one-launch solve in this precision, built on its first use for the mesh; none (groups == 0)
 // when the operator does not fit the chip.
 void ensure_resident(fem_ctx* c, bool fp32) {
-    if (c->res_precision == (fp32 ? 1 : 0)) return;
-    c->res = ResidentTables{};
-    c->res_precision = fp32 ? 1 : 0;
-    c->res_columns = 1;
+    Resident& r = c->res[fp32];
+    if (r.planned) return;
+    r.planned = true;
+    r.t = ResidentTables{};
+    r.columns = 1;
     if (c->cg_kernels != 0 || c->kind == FEM_ELEMENT_HEX) return;
     const ResidentPlan plan =
         c->num_instances > 0 ? plan_resident_batch(c->h_node_off, c->h_rowptr_b.data(), c->h_colidx_b.data(),
@@ -525,34 +531,34 @@ void ensure_resident(fem_ctx* c, bool fp32) {
     add(plan.row_lane);
     add(plan.cols);
     add(plan.wg);
-    c->res_mem.alloc(h.size());
-    c->res_mem.upload(h.data(), h.size(), c->stream);
+    r.mem.alloc(h.size());
+    r.mem.upload(h.data(), h.size(), c->stream);
     // columns of a compliance solve (FP64) go side by side while CUs are left
     if (c->num_instances == 0 && !fp32)
-        c->res_columns = std::max(1, std::min(kResMaxColumns, std::min(c->num_cus, kResMaxGroups) / plan.groups));
-    c->res_exch.alloc(2 * (size_t)c->res_columns * c->num_nodes * (fp32 ? kResRowBytes32 : kResRowBytes64));
-    c->res_dirty = true;
-    c->res_slots.alloc(kResSlotWords * std::max<size_t>(1, plan.launches.size()));
-    c->res_launches = plan.launches;
-    c->res_instances = plan.instances;
+        r.columns = std::max(1, std::min(kResMaxColumns, std::min(c->num_cus, kResMaxGroups) / plan.groups));
+    r.exch.alloc(2 * (size_t)r.columns * c->num_nodes * (fp32 ? kResRowBytes32 : kResRowBytes64));
+    r.dirty = true;
+    r.slots.alloc(kResSlotWords * std::max<size_t>(1, plan.launches.size()));
+    r.launches = plan.launches;
+    r.instances = plan.instances;
     HIPCHECK(hipStreamSynchronize(c->stream));
-    unsigned char* p = c->res_mem.p;
-    c->res.nb = plan.nb;
-    c->res.rows = (int)c->num_nodes;
-    c->res.group = reinterpret_cast<const int4*>(p + at[0]);
-    c->res.row_node = reinterpret_cast<const int*>(p + at[1]);
-    c->res.halo_node = reinterpret_cast<const int*>(p + at[2]);
-    c->res.halo_pos = reinterpret_cast<const int*>(p + at[3]);
-    c->res.lane_k0 = reinterpret_cast<const int*>(p + at[4]);
-    c->res.lane_info = reinterpret_cast<const int*>(p + at[5]);
-    c->res.row_lane = reinterpret_cast<const uint16_t*>(p + at[6]);
-    c->res.cols = reinterpret_cast<const uint16_t*>(p + at[7]);
-    c->res.wg = c->num_instances > 0 ? reinterpret_cast<const int4*>(p + at[8]) : nullptr;
-    c->res.groups = plan.groups;
+    unsigned char* p = r.mem.p;
+    r.t.nb = plan.nb;
+    r.t.rows = (int)c->num_nodes;
+    r.t.group = reinterpret_cast<const int4*>(p + at[0]);
+    r.t.row_node = reinterpret_cast<const int*>(p + at[1]);
+    r.t.halo_node = reinterpret_cast<const int*>(p + at[2]);
+    r.t.halo_pos = reinterpret_cast<const int*>(p + at[3]);
+    r.t.lane_k0 = reinterpret_cast<const int*>(p + at[4]);
+    r.t.lane_info = reinterpret_cast<const int*>(p + at[5]);
+    r.t.row_lane = reinterpret_cast<const uint16_t*>(p + at[6]);
+    r.t.cols = reinterpret_cast<const uint16_t*>(p + at[7]);
+    r.t.wg = c->num_instances > 0 ? reinterpret_cast<const int4*>(p + at[8]) : nullptr;
+    r.t.groups = plan.groups;
 }
 
 bool use_resident(const fem_ctx* c, bool fp32) {
-    return c->res.groups > 0 && c->res_precision == (fp32 ? 1 : 0) && c->res_backoff == 0;
+    return fp32 == (c->opt.precision == FEM_PRECISION_FP32_REFINED) && c->res[fp32].t.groups > 0 && c->res_backoff == 0;
 }
 
 constexpr int kResBackoff = 256;  // solves with one launch per iteration after a one-launch solve gave up
@@ -566,21 +572,28 @@ ChipShare::Use share_chip(const fem_ctx* c, int workgroups) {
     return ChipShare::Use(chips[(unsigned)c->device % 64], workgroups, c->num_cus);
 }
 
-ResidentArgs resident_args(fem_ctx* c) {
-    if (c->res_dirty) {
-        HIPCHECK(hipMemsetAsync(c->res_exch.p, 0, c->res_exch.n, c->stream));
-        c->res_dirty = false;
+ResidentArgs resident_args(fem_ctx* c, bool fp32) {
+    Resident& res = c->res[fp32];
+    if (res.dirty) {
+        HIPCHECK(hipMemsetAsync(res.exch.p, 0, res.exch.n, c->stream));
+        res.dirty = false;
     }
     ResidentArgs r;
-    r.t = c->res;
-    r.exch = c->res_exch.p;
-    r.slots = c->res_slots.p;
+    r.t = res.t;
+    r.exch = res.exch.p;
+    r.slots = res.slots.p;
     r.wait_ticks = c->res_wait_ticks;
     return r;
 }
 
+// A one-launch solve gave up waiting: it is done again with a launch per iteration, as are the next solves.
+void resident_gave_up(fem_ctx* c, bool fp32) {
+    c->res_backoff = kResBackoff;
+    c->res[fp32].dirty = true;
+}
+
 void launch_resident(fem_ctx* c, const CgArgs& a, int max_iter) {
-    ResidentArgs r = resident_args(c);
+    ResidentArgs r = resident_args(c, a.fp32);
     r.S = a.S;
     r.r = a.r1;
     r.z = a.z1;
@@ -614,7 +627,7 @@ CgArgs cg_args(fem_ctx* c, bool fp32, double tol) {
     a.w[1] = c->cg_w1.p;
     a.part7 = c->part7.p;
     a.binv = c->cg_binv.p;
-    a.slots = use_resident(c, fp32) ? c->res_slots.p : nullptr;
+    a.slots = use_resident(c, fp32) ? c->res[fp32].slots.p : nullptr;
     return a;
 }
 
@@ -663,7 +676,7 @@ int64_t max_iters(fem_ctx* c) {
 int run_cg_iterations(fem_ctx* c, const CgArgs& a, const double* b, int max_iter) {
     int& pred = c->solving_adjoint ? c->predicted_adj : c->predicted_iters;
     if (a.slots) {
-        const ChipShare::Use cus = share_chip(c, c->res.groups);
+        const ChipShare::Use cus = share_chip(c, c->res[a.fp32].t.groups);
         TIMED(c, FEM_PHASE_SPMV, 0, launch_resident(c, a, max_iter));
         HIPCHECK(hipMemcpyAsync(c->h_sc, a.sc, sizeof(CgScalars), hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(hipStreamSynchronize(c->stream));
@@ -672,9 +685,7 @@ int run_cg_iterations(fem_ctx* c, const CgArgs& a, const double* b, int max_iter
             pred = c->h_sc->iters + 1;
             return c->h_sc->iters;
         }
-        // gave up waiting for a workgroup: started over with one launch per iteration, as are the next solves
-        c->res_backoff = kResBackoff;
-        c->res_dirty = true;
+        resident_gave_up(c, a.fp32);
         CgArgs t = a;
         t.slots = nullptr;
         launch_solver_init(c, t, b, nullptr);
@@ -786,7 +797,7 @@ void linear_solve(fem_ctx* c) {
     a.floor_tol = kInnerFloor * c->opt.cg_tolerance;
     if (max_iter < 1) a.slots = nullptr;
     ChipShare::Use cus;
-    if (a.slots) cus = share_chip(c, c->res.groups);
+    if (a.slots) cus = share_chip(c, c->res[a.fp32].t.groups);
     CgScalars* outer = c->scal.p + 1;
     // One-kernel CG path: sweep s is one launch for dv_s = dv_{s-1} + x_{s-1}, the FP64 residual and the inner
     // solve's start, and one for the outer test with the inner scalars; dv_s and x_s alternate between two
@@ -856,9 +867,8 @@ void linear_solve(fem_ctx* c) {
         read_back(sweep);
     }
     if (a.slots && c->h_sc[1].pad) {
-        // an inner solve gave up waiting for a workgroup: the solve starts over with one launch per iteration
-        c->res_backoff = kResBackoff;
-        c->res_dirty = true;
+        // in an inner solve: the whole refinement starts over
+        resident_gave_up(c, true);
         cus.release();
         return linear_solve(c);
     }
@@ -1272,8 +1282,8 @@ BatchCg batch_args(fem_ctx* c, bool fp32) {
     a.kA = c->b_kA.p;
     a.kV = c->b_kV.p;
     if (use_resident(c, fp32) && c->opt.cg_max_iterations != 0) {
-        a.slots = c->res_slots.p;
-        a.slot_words = c->res_slots.n;
+        a.slots = c->res[fp32].slots.p;
+        a.slot_words = c->res[fp32].slots.n;
     }
     return a;
 }
@@ -1357,8 +1367,9 @@ int run_batch_solves(fem_ctx* c, const BatchCg& a, const double* b, const CgScal
     const int M = c->num_instances;
     bool gave_up = false, rest = false;
     {
-        const ChipShare::Use cus = share_chip(c, *std::max_element(c->res_launches.begin(), c->res_launches.end()));
-        ResidentArgs r = resident_args(c);
+        const std::vector<int>& launches = c->res[a.fp32].launches;
+        const ChipShare::Use cus = share_chip(c, *std::max_element(launches.begin(), launches.end()));
+        ResidentArgs r = resident_args(c, a.fp32);
         r.S = a.S;
         r.r = a.r;
         r.z = a.z;
@@ -1367,7 +1378,7 @@ int run_batch_solves(fem_ctx* c, const BatchCg& a, const double* b, const CgScal
         r.sc = a.sc;
         r.max_iter = 0;
         r.max_iters = a.t.inst_maxit;
-        for (int wgs : c->res_launches) {
+        for (int wgs : launches) {
             launch_cg_resident(r, a.fp32, c->stream, wgs);
             r.t.wg += wgs;
             r.slots += kResSlotWords;
@@ -1378,12 +1389,11 @@ int run_batch_solves(fem_ctx* c, const BatchCg& a, const double* b, const CgScal
     int mx = 0;
     for (int i = 0; i < M; ++i) {
         gave_up = gave_up || c->h_bsc[i].pad;
-        rest = rest || (!c->res_instances[i] && !c->h_bsc[i].done);
+        rest = rest || (!c->res[a.fp32].instances[i] && !c->h_bsc[i].done);
         mx = std::max(mx, c->h_bsc[i].iters);
     }
     if (gave_up) {
-        c->res_backoff = kResBackoff;
-        c->res_dirty = true;
+        resident_gave_up(c, a.fp32);
         BatchCg t = a;
         t.slots = nullptr;
         t.slot_words = 0;
@@ -2529,17 +2539,18 @@ ColumnWork column_work(double* base, CgScalars* sc, size_t n, int columns) {
     return {base, base + columns * n, base + 2 * columns * n, base + (2 * columns + 1) * n, sc};
 }
 
-// Columns [0, ncols) of b through the one-launch CG, c->res_columns side by side; x is written in place in out, with the
+// Columns [0, ncols) of b through the one-launch CG, as many side by side as the chip holds; x is written in place in out, with the
 // boundary rows zero from the start. False when a solve gave up waiting (out is then solved again by the caller).
 bool resident_columns(fem_ctx* c, const double* b, int64_t ncols, double* out, const ColumnWork& w) {
     const size_t n = (size_t)c->ndof;
     CgScalars h[kResColumnStates];
-    const ChipShare::Use cus = share_chip(c, c->res.groups * (int)std::min<int64_t>(c->res_columns, ncols));
+    const Resident& res = c->res[0];
+    const ChipShare::Use cus = share_chip(c, res.t.groups * (int)std::min<int64_t>(res.columns, ncols));
     for (int64_t j0 = 0; j0 < ncols; j0 += kResColumnStates) {
         const int some = (int)std::min<int64_t>(kResColumnStates, ncols - j0);
-        for (int j = 0; j < some; j += c->res_columns) {
-            const int cnt = std::min(c->res_columns, some - j);
-            ResidentArgs r = resident_args(c);
+        for (int j = 0; j < some; j += res.columns) {
+            const int cnt = std::min(res.columns, some - j);
+            ResidentArgs r = resident_args(c, false);
             r.S = c->S64.p;
             r.r = w.r;
             r.z = w.z;
@@ -2551,15 +2562,14 @@ bool resident_columns(fem_ctx* c, const double* b, int64_t ncols, double* out, c
             r.stride = (int64_t)n;
             launch_resident_columns((int)c->num_nodes, cnt, b + (j0 + j) * n, c->bcmask.p, c->diagblk.p, c->S64.p,
                                     c->opt.cg_tolerance, out + (j0 + j) * n, w.r, w.z, w.dinv, w.partial, w.sc + j,
-                                    c->res_slots.p, c->stream);
+                                    res.slots.p, c->stream);
             launch_cg_resident(r, false, c->stream);
         }
         HIPCHECK(hipMemcpyAsync(h, w.sc, some * sizeof(CgScalars), hipMemcpyDeviceToHost, c->stream));
         HIPCHECK(hipStreamSynchronize(c->stream));
         for (int j = 0; j < some; ++j)
             if (h[j].pad) {
-                c->res_backoff = kResBackoff;
-                c->res_dirty = true;
+                resident_gave_up(c, false);
                 return false;
             }
     }
@@ -2608,10 +2618,10 @@ void compliance_tet(fem_ctx* c, const double* b, int64_t ncols, double* out) {
         }
     }
     if (use_resident_columns(c, b, out, ncols)) {
-        const size_t need = column_work_doubles(n, c->res_columns);
+        const size_t need = column_work_doubles(n, c->res[0].columns);
         if (c->res_col.n < need) c->res_col.alloc(need);
         if (!c->res_col_sc.p) c->res_col_sc.alloc(kResColumnStates);
-        if (resident_columns(c, b, ncols, out, column_work(c->res_col.p, c->res_col_sc.p, n, c->res_columns))) return;
+        if (resident_columns(c, b, ncols, out, column_work(c->res_col.p, c->res_col_sc.p, n, c->res[0].columns))) return;
     }
     if (c->mcg_b.n != n * 8) {
         for (DevBuf<double>* v : {&c->mcg_b, &c->mcg_x, &c->mcg_r, &c->mcg_z, &c->mcg_p, &c->mcg_q}) v->alloc(n * 8);
@@ -2710,11 +2720,11 @@ int fem_apply_compliance_device_noalloc(fem_ctx* c, const double* b, int64_t num
             compliance_lu(c, b, num_columns, out, (double*)base, tc);
             return FEM_OK;
         }
-        const size_t work = column_work_doubles((size_t)c->ndof, c->res_columns) * sizeof(double);
+        const size_t work = column_work_doubles((size_t)c->ndof, c->res[0].columns) * sizeof(double);
         const size_t work_up = (work + 255) & ~size_t(255);
         if (use_resident_columns(c, b, out, num_columns) && work_up + kResColumnStates * sizeof(CgScalars) <= kNoAllocScratchBytes &&
             resident_columns(c, b, num_columns, out,
-                             column_work((double*)base, (CgScalars*)(base + work_up), (size_t)c->ndof, c->res_columns)))
+                             column_work((double*)base, (CgScalars*)(base + work_up), (size_t)c->ndof, c->res[0].columns)))
             return FEM_OK;
         McgColumn status[8];
         const McgWork w{(double*)(base + L.b), (double*)(base + L.x), (double*)(base + L.r),
@@ -3132,8 +3142,10 @@ int fem_set_instances(fem_ctx* c, int32_t num_instances, const int64_t* node_off
             ei[e] = i;
         }
         c->num_instances = M;
-        c->res_precision = -1;  // planned per instance at the next solve
-        c->res = ResidentTables{};
+        for (Resident& r : c->res) {  // planned per instance at the next solve
+            r.planned = false;
+            r.t = ResidentTables{};
+        }
         c->linear_matrix_ready = false;
         c->elem_inst.alloc(c->num_elements);
         c->elem_inst.upload(ei.data(), c->num_elements, c->stream);

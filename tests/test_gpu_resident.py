@@ -157,6 +157,41 @@ def test_repeats_bit_for_bit_and_from_threads(monkeypatch):
         assert np.array_equal(w[0], g[0]) and np.array_equal(w[1], g[1])
 
 
+def test_changes_between_precisions(monkeypatch):
+    """A context that changes between FP64 and FP32 + refinement: FP64 frames are those of a context that stays in FP64 bit for
+    bit, and only the first change to each waits for its partition of the mesh on the host (3 ms and more at this size, a later
+    change 0.1 ms)."""
+    monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+    x0, tets, bc = block((40, 40, 40))
+    v0 = 0.01 * np.random.RandomState(1).standard_normal(x0.size)
+    g, h = femgpu.FemGpu(0), femgpu.FemGpu(0)
+    for c in (g, h):
+        c.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets, 5e4, 0.4, 1000.0)
+        c.add_bc_nodes(bc)
+    h.set_options(dt=1e-3, cg_tolerance=TOL, precision=femgpu.FP64)
+    h.set_state(x0, v0)
+    assert h.step(1) == femgpu.FEM_OK
+    want = h.state()
+    took = []
+    for _ in range(5):
+        took.append(0.0)
+        for precision in (femgpu.FP64, femgpu.FP32_REFINED):
+            t0 = time.perf_counter()
+            g.set_options(dt=1e-3, cg_tolerance=TOL, precision=precision)
+            took[-1] += time.perf_counter() - t0
+            g.set_state(x0, v0)
+            assert g.step(1) == femgpu.FEM_OK
+            x, v = g.state()
+            if precision == femgpu.FP64:
+                assert np.array_equal(x, want[0]) and np.array_equal(v, want[1])
+            else:
+                assert np.linalg.norm(v - want[1]) <= BOUND * np.linalg.norm(want[1])
+    print("two changes: %s ms" % " ".join("%.2f" % (1e3 * t) for t in took), flush=True)
+    assert min(took[1:]) < 0.5 * took[0]
+    g.close()
+    h.close()
+
+
 def test_small_body_beside_a_long_solve():
     """A body of 4 workgroups steps beside one of 25 whose solves take hundreds of iterations, on its own stream from another
     thread: it does not wait for the other's solve to end. Its median frame is held to half of the other's; it took 0.16 of it
