@@ -404,8 +404,8 @@ __device__ __forceinline__ void hex_products(const float4* Ct, const float (&pv)
         }
         // The next group's loads take their address from a value this group produced (a zero the compiler
         // cannot see through), so they are not hoisted above this group's products: without it the compiler
-        // keeps most of the 75 chunks in flight at once (over 300 registers, 1 wave per SIMD) instead of about
-        // two groups (210 registers, 2 waves per SIMD).
+        // may keep most of the 75 chunks in flight at once (over 300 registers, 1 wave per SIMD) instead of
+        // about two groups (96 registers with TABLE, 111 without: 5 and 4 waves per SIMD).
         {
             int zero;
             asm volatile("v_mov_b32 %0, 0" : "=v"(zero) : "v"(y[3 * kOff.b[4 * g + 3] + 2]));
@@ -436,48 +436,14 @@ __device__ __forceinline__ void hex_products(const float4* Ct, const float (&pv)
     }
 }
 
-// The same products in the same order with one matrix for every lane: its 300 floats lie across the lanes of 5 registers and
-// are read back one by one as scalars (v_readlane). The products then wait for no load; through scalar loads they took 9.5 us
-// at 64x33x65 cubes, each load a wait of its own, with 2 waves on a SIMD to hide it.
-__device__ __forceinline__ void hex_products_scalar(const float (&held)[5], const float (&pv)[24], float (&y)[24]) {
-    auto at = [&](int f) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, held[f >> 6]), f & 63));
-    };
-#pragma unroll
-    for (int a = 0; a < 8; ++a)
-#pragma unroll
-        for (int b = a + 1; b < 8; ++b) {
-            float B[9];
-#pragma unroll
-            for (int i = 0; i < 9; ++i) B[i] = at(9 * off_index(a, b) + i);
-#pragma unroll
-            for (int i = 0; i < 3; ++i)
-                y[3 * a + i] += B[3 * i] * pv[3 * b] + B[3 * i + 1] * pv[3 * b + 1] + B[3 * i + 2] * pv[3 * b + 2];
-#pragma unroll
-            for (int j = 0; j < 3; ++j)
-                y[3 * b + j] += B[j] * pv[3 * a] + B[3 + j] * pv[3 * a + 1] + B[6 + j] * pv[3 * a + 2];
-        }
-#pragma unroll
-    for (int a = 0; a < 8; ++a) {
-        float B[6];
-#pragma unroll
-        for (int i = 0; i < 6; ++i) B[i] = at(kHexOffFloats + 6 * a + i);
-        const float p0 = pv[3 * a], p1 = pv[3 * a + 1], p2 = pv[3 * a + 2];
-        y[3 * a] += B[0] * p0 + B[1] * p1 + B[2] * p2;
-        y[3 * a + 1] += B[1] * p0 + B[3] * p1 + B[4] * p2;
-        y[3 * a + 2] += B[2] * p0 + B[4] * p1 + B[5] * p2;
-    }
-}
-
 // FP32 cached operator: stage = A_e p_e of every element, one element per lane, with p = z + beta p_old of CG iteration k
 // formed on the fly (sc null: p as it is). p is zero on BC DOFs without
 // a mask: hex_cg_init_kernel zeroes r there, and the BC rows of the operator are the identity (q = p on them),
-// so r, z and p stay zero on those rows through the solve. kTable: A_e is entry table_idx[t] of the
-// distinct-matrix table, staged in LDS by every workgroup. kOneMatrix: the table has one entry, which comes as scalars:
-// the products read their factors from scalar registers, so that a lane holds 76 vector registers instead of 192 and 6 waves
-// run on a SIMD instead of 2. The same floats and the same arithmetic in every case.
-enum HexSource { kPerPosition, kTable, kOneMatrix };
-template <HexSource SOURCE>
+// so r, z and p stay zero on those rows through the solve. TABLE: A_e is entry table_idx[t] of the
+// distinct-matrix table, staged in LDS by every workgroup. The same floats and the same arithmetic in both cases.
+// A single matrix goes through the table too: held across a wave's lanes and read back as scalars, it took 1.26 ms a step at
+// 64x33x65 cubes against 1.22 (0.89 against 0.89 at 40^3, 4.5 against 4.6 at 128x64x128).
+template <bool TABLE>
 __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const int* __restrict__ order_pad,
                                                           const int* __restrict__ conn,
                                                           const float4* __restrict__ A4,
@@ -492,14 +458,6 @@ __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const i
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     const int e = t < count_pad ? order_pad[t] : -1;
     HexCgStart start(sc ? k : 0, partial);
-    float held[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
-    if constexpr (SOURCE == kOneMatrix) {
-#pragma unroll
-        for (int i = 0; i < 5; ++i) {
-            const int f = 64 * i + (threadIdx.x & 63);
-            held[i] = reinterpret_cast<const float*>(table)[f < 4 * kHexChunks ? f : 0];
-        }
-    }
     if (sc && sc->done) return;  // no scalars when the operator is timed alone
     float pv[24], y[24];
     // the element's inputs are on their way while the block sums of the last iteration are added up
@@ -516,19 +474,18 @@ __global__ __launch_bounds__(256) void hex_apply32_kernel(int count_pad, const i
                 if (sc) y[3 * a + c] = z[d];
             }
     }
-    if (SOURCE == kTable)
+    if (TABLE)
         for (int i = threadIdx.x; i < num_distinct * kHexChunks; i += blockDim.x) lds_table[i] = table[i];
     double beta = 0.0;
     if (sc && !start.finish(k, max_iter, sc, beta, lds)) return;
-    if (SOURCE == kTable) __syncthreads();
+    if (TABLE) __syncthreads();
     if (e < 0) return;
 #pragma unroll
     for (int j = 0; j < 24; ++j) {
         if (sc) pv[j] = k > 0 ? y[j] + (float)beta * pv[j] : y[j];
         y[j] = 0.f;
     }
-    if constexpr (SOURCE == kOneMatrix) hex_products_scalar(held, pv, y);
-    else if constexpr (SOURCE == kTable) hex_products<true>(lds_table + table_idx[t] * kHexChunks, pv, y);
+    if constexpr (TABLE) hex_products<true>(lds_table + table_idx[t] * kHexChunks, pv, y);
     else hex_products<false>(A4 + (size_t)(t >> 6) * kHexChunks * 64 + (t & 63), pv, y);
     float* st = stage + stage_at(t);
 #pragma unroll
@@ -1109,9 +1066,8 @@ void elements32(const HexData& h, const float* p, const HexIteration<float>& it,
                            reinterpret_cast<const float4*>(h.table), h.table_idx, h.num_distinct, p, (float*)h.stage,
                            it.k, it.max_iter, it.z, (const double*)it.partial, it.sc);
     };
-    if (h.num_distinct == 1) launch(hex_apply32_kernel<kOneMatrix>, 0);
-    else if (h.num_distinct > 1) launch(hex_apply32_kernel<kTable>, (size_t)h.num_distinct * kHexChunks * sizeof(float4));
-    else launch(hex_apply32_kernel<kPerPosition>, 0);
+    if (h.num_distinct > 0) launch(hex_apply32_kernel<true>, (size_t)h.num_distinct * kHexChunks * sizeof(float4));
+    else launch(hex_apply32_kernel<false>, 0);
 }
 
 // y = y_in + sign (am M + ak K) w (FP64, matrix-free).

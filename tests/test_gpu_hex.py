@@ -112,7 +112,7 @@ def test_hex_distinct_matrix_table(monkeypatch):
 
 @pytest.mark.parametrize("moduli", [1, 2, 32, 33])
 def test_hex_operator_by_number_of_matrices(moduli, monkeypatch):
-    """One distinct matrix (kept in registers), a few (the table, to its limit of 32) and more (one per element) on an odd-sized
+    """One distinct matrix and a few (the table, to its limit of 32) and more (one per element) on an odd-sized
     block of 525 elements, which ends in a part-filled tile: the same floats in the same order, so the trajectory is that of the
     per-element cache bit for bit."""
     cfg = mg.config_hex((7, 5, 15))
