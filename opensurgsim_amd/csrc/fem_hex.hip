@@ -374,7 +374,7 @@ __global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slot
 }
 
 // y += A_e p_e from an element's 75 chunks at Ct, one after another (SHARED: in LDS) or 64 apart. The 36 blocks stream in 9
-// groups of 4 (36 floats = 9 float4 chunks per group).
+// groups of 4 (36 floats = 9 float4 chunks per group); a lane holds 96 registers (SHARED) or 107, 5 or 4 waves on a SIMD.
 template <bool SHARED>
 __device__ __forceinline__ void hex_products(const float4* Ct, const float (&pv)[24], float (&y)[24]) {
     constexpr size_t kStep = SHARED ? 1 : 64;
@@ -401,15 +401,6 @@ __device__ __forceinline__ void hex_products(const float4* Ct, const float (&pv)
 #pragma unroll
             for (int j = 0; j < 3; ++j)
                 y[3 * b + j] += B[j] * pv[3 * a] + B[3 + j] * pv[3 * a + 1] + B[6 + j] * pv[3 * a + 2];
-        }
-        // The next group's loads take their address from a value this group produced (a zero the compiler
-        // cannot see through), so they are not hoisted above this group's products: without it the compiler
-        // may keep most of the 75 chunks in flight at once (over 300 registers, 1 wave per SIMD) instead of
-        // about two groups (96 registers with TABLE, 111 without: 5 and 4 waves per SIMD).
-        {
-            int zero;
-            asm volatile("v_mov_b32 %0, 0" : "=v"(zero) : "v"(y[3 * kOff.b[4 * g + 3] + 2]));
-            Ct += zero;
         }
     }
     // the diagonal blocks, 4 per group of 6 chunks (symmetric, 6 floats each)
