@@ -301,24 +301,27 @@ __global__ __launch_bounds__(128, 2) void hex_apply64_kernel(int count_pad, cons
 }
 
 // y = y_in + sign * (the staged values of each node's elements, in colour order) (y_in null: 0). src[slot * num_nodes + node]:
-// where the node's values of its slot-th element start (-1: none). With sc (CG iteration k, the element kernel of which
+// where the node's values of its slot-th element start (kNotStaged: none), for at most kStageSlots elements; those of the elements
+// past them are at more[more_ptr[node]] to more[more_ptr[node + 1]] (more_ptr null: no node has any). With sc (CG iteration k, the element kernel of which
 // formed p = z + beta p on the fly): p is stored, the BC rows of the operator are the identity (y = p), and
 // with pq the partial p . y goes to slot 2 of the partials.
 template <typename TV>
-__global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slots, const int* __restrict__ src,
+__global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slots, const uint32_t* __restrict__ src,
+                                                         const int64_t* __restrict__ more_ptr,
+                                                         const uint32_t* __restrict__ more,
                                                          const TV* __restrict__ stage, TV sign, const TV* y_in, TV* y,
                                                          int k, const TV* __restrict__ z, TV* __restrict__ p,
                                                          const uint8_t* __restrict__ mask, int pq,
                                                          double* __restrict__ partial, const CgScalars* __restrict__ sc) {
     __shared__ double lds[64];
     const int first = blockIdx.x * blockDim.x + threadIdx.x;
-    int at[8];  // the node's first staged values, asked for ahead of the scalars
-    auto ask = [&](int i, int b) {
+    uint32_t at[kStageSlots];  // where the node's values are staged, asked for ahead of the scalars
+    auto ask = [&](int i) {
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            at[u] = i < num_nodes && b + u < slots ? src[(int64_t)(b + u) * num_nodes + i] : -1;
+        for (int u = 0; u < kStageSlots; ++u)
+            at[u] = i < num_nodes && u < slots ? src[(int64_t)u * num_nodes + i] : kNotStaged;
     };
-    ask(first, 0);
+    ask(first);
     if (sc && sc->done) return;
     const TV beta = sc && k > 0 ? (TV)(sc->rz[k & 1] / sc->rz[(k - 1) & 1]) : TV(0);
     double acc = 0.0;
@@ -338,20 +341,29 @@ __global__ __launch_bounds__(512) void hex_gather_kernel(int num_nodes, int slot
             s1 = y_in[3 * (int64_t)i + 1];
             s2 = y_in[3 * (int64_t)i + 2];
         }
-        for (int b = 0; b < slots; b += 8) {
-            if (b > 0 || i != first) ask(i, b);
-            TV g[8][3];
+        auto add = [&] {
+            TV g[kStageSlots][3];
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < kStageSlots; ++u)
 #pragma unroll
-                for (int c = 0; c < 3; ++c) g[u][c] = at[u] >= 0 ? stage[(int64_t)at[u] + 64 * c] : TV(0);
+                for (int c = 0; c < 3; ++c) g[u][c] = at[u] != kNotStaged ? stage[(int64_t)at[u] + 64 * c] : TV(0);
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (at[u] >= 0) {
+            for (int u = 0; u < kStageSlots; ++u)
+                if (at[u] != kNotStaged) {
                     s0 += sign * g[u][0];
                     s1 += sign * g[u][1];
                     s2 += sign * g[u][2];
                 }
+        };
+        if (i != first) ask(i);
+        add();
+        if (more_ptr) {
+            const int64_t end = more_ptr[i + 1];
+            for (int64_t j = more_ptr[i]; j < end; j += kStageSlots) {
+#pragma unroll
+                for (int u = 0; u < kStageSlots; ++u) at[u] = j + u < end ? more[j + u] : kNotStaged;
+                add();
+            }
         }
         TV s[3] = {s0, s1, s2};
         if (sc) {
@@ -802,7 +814,7 @@ double host_hex_volume(const double* X, int64_t e) {
 void hex_release(HexData& h) {
     for (void* p : {(void*)h.conn, (void*)h.order, (void*)h.order_pad, (void*)h.A32, (void*)h.diag64, (void*)h.diag32,
                     (void*)h.table, (void*)h.table_idx, (void*)h.mdiag_cons, (void*)h.mdiag_lump, (void*)h.diagx64,
-                    (void*)h.diagx32, (void*)h.stage, (void*)h.src})
+                    (void*)h.diagx32, (void*)h.stage, (void*)h.src, (void*)h.more_ptr, (void*)h.more})
         if (p) (void)hipFree(p);
     h.mdiag_cons = h.mdiag_lump = nullptr;
     h.diagx64 = nullptr;
@@ -812,11 +824,38 @@ void hex_release(HexData& h) {
     h.table_idx = nullptr;
     h.num_distinct = 0;
     h.stage = nullptr;
-    h.src = nullptr;
+    h.src = h.more = nullptr;
+    h.more_ptr = nullptr;
     h.A32 = nullptr;
     h.diag64 = nullptr;
     h.diag32 = nullptr;
     h.ready = false;
+}
+
+HexStageMap hex_stage_map(int64_t num_nodes, const int32_t* conn, const std::vector<int>& order_pad) {
+    if (24 * order_pad.size() > (size_t)kNotStaged) throw std::invalid_argument("mesh too large for 32-bit staging offsets");
+    HexStageMap m;
+    std::vector<int> cnt(num_nodes, 0);
+    for (int e : order_pad)
+        if (e >= 0)
+            for (int a = 0; a < 8; ++a) m.slots = std::max(m.slots, ++cnt[conn[8 * (size_t)e + a]]);
+    if (m.slots > kStageSlots) {
+        m.slots = kStageSlots;
+        m.more_ptr.assign(num_nodes + 1, 0);
+        for (int64_t i = 0; i < num_nodes; ++i) m.more_ptr[i + 1] = m.more_ptr[i] + std::max(0, cnt[i] - kStageSlots);
+        m.more.resize(m.more_ptr[num_nodes]);
+    }
+    m.src.assign((size_t)m.slots * num_nodes, kNotStaged);
+    std::fill(cnt.begin(), cnt.end(), 0);
+    for (size_t t = 0; t < order_pad.size(); ++t)
+        if (order_pad[t] >= 0)
+            for (int a = 0; a < 8; ++a) {
+                const int i = conn[8 * (size_t)order_pad[t] + a], k = cnt[i]++;
+                const uint32_t at = (uint32_t)((t / 64) * 24 * 64 + (size_t)(3 * a) * 64 + t % 64);
+                if (k < kStageSlots) m.src[(size_t)k * num_nodes + i] = at;
+                else m.more[m.more_ptr[i] + k - kStageSlots] = at;
+            }
+    return m;
 }
 
 void hex_setup(HexData& h, int64_t num_nodes, const double* x0, int64_t num_elements, const int32_t* conn,
@@ -885,22 +924,17 @@ void hex_setup(HexData& h, int64_t num_nodes, const double* x0, int64_t num_elem
     std::vector<int> order_pad(h.pad_ptr[ncol], -1);
     for (int c = 0; c < ncol; ++c)
         std::copy(order.begin() + h.color_ptr[c], order.begin() + h.color_ptr[c + 1], order_pad.begin() + h.pad_ptr[c]);
-    // where each node's values of its elements are staged, in colour order (= the padded order)
-    h.slots = 0;
     {
-        std::vector<int> cnt(num_nodes, 0);
-        for (int64_t i = 0; i < 8 * num_elements; ++i) h.slots = std::max(h.slots, ++cnt[conn[i]]);
-        if (24 * order_pad.size() > (size_t)INT32_MAX) throw std::invalid_argument("mesh too large for int32 staging offsets");
-        std::vector<int> src((size_t)h.slots * num_nodes, -1);
-        std::fill(cnt.begin(), cnt.end(), 0);
-        for (size_t t = 0; t < order_pad.size(); ++t)
-            if (order_pad[t] >= 0)
-                for (int a = 0; a < 8; ++a) {
-                    const int i = conn[8 * (size_t)order_pad[t] + a];
-                    src[(size_t)cnt[i]++ * num_nodes + i] = (int)((t / 64) * 24 * 64 + (size_t)(3 * a) * 64 + t % 64);
-                }
-        HCHECK(hipMalloc(&h.src, src.size() * sizeof(int)));
-        HCHECK(hipMemcpyAsync(h.src, src.data(), src.size() * sizeof(int), hipMemcpyHostToDevice, s));
+        const HexStageMap map = hex_stage_map(num_nodes, conn, order_pad);
+        h.slots = map.slots;
+        auto put = [&](auto*& to, const auto& from) {
+            if (from.empty()) return;
+            HCHECK(hipMalloc(&to, from.size() * sizeof(from[0])));
+            HCHECK(hipMemcpyAsync(to, from.data(), from.size() * sizeof(from[0]), hipMemcpyHostToDevice, s));
+        };
+        put(h.src, map.src);
+        put(h.more_ptr, map.more_ptr);
+        put(h.more, map.more);
         HCHECK(hipStreamSynchronize(s));
         HCHECK(hipMalloc(&h.stage, order_pad.size() * 24 * sizeof(double)));
     }
@@ -1026,7 +1060,7 @@ struct HexIteration {
 template <typename TV>
 void gather(const HexData& h, TV sign, const TV* y_in, TV* y, const HexIteration<TV>& it, hipStream_t s) {
     hipLaunchKernelGGL((hex_gather_kernel<TV>), dim3(kCgBlocks), dim3(512), 0, s, (int)h.num_nodes, h.slots, h.src,
-                       (const TV*)h.stage, sign, y_in, y, it.k, it.z, it.p, it.mask, it.pq, it.partial,
+                       h.more_ptr, h.more, (const TV*)h.stage, sign, y_in, y, it.k, it.z, it.p, it.mask, it.pq, it.partial,
                        (const CgScalars*)it.sc);
 }
 

@@ -27,8 +27,10 @@ struct HexData {
     std::vector<int> pad_ptr;     // colour c: order_pad[pad_ptr[c] .. pad_ptr[c + 1]), multiples of 64
     int* order_pad = nullptr;     // colour order padded to 64-element tiles (-1 = padding)
     void* stage = nullptr;        // staged products of an application, 24 values per padded position (see fem_hex.hip)
-    int* src = nullptr;           // [slots][num_nodes] where each node's values are staged, colour order (-1: none)
-    int slots = 0;                // most elements of a node
+    uint32_t* src = nullptr;      // HexStageMap on the device
+    int64_t* more_ptr = nullptr;
+    uint32_t* more = nullptr;
+    int slots = 0;
     float* A32 = nullptr;         // packed upper triangle of M/dt + dt K (FP32): 28 upper node blocks of 9 and
                                   // 8 symmetric diagonal blocks of 6, 300 floats per padded position,
                                   // interleaved by 64-position tiles in float4 chunks
@@ -50,6 +52,20 @@ struct HexData {
     int predicted_sweeps = 0;           // refinement sweeps of the last solve
     bool ready = false;
 };
+
+// Where each node's values of its elements are staged, in the order of the padded positions (colour order). 32-bit offsets: the
+// largest mesh (2^27 elements) stages 24 x 2^27 values. A node of a block has at most 8 elements; the few nodes of an
+// unstructured mesh that have more keep the rest in a list, so that one node of very many elements costs no more than these.
+constexpr int kStageSlots = 8;
+constexpr uint32_t kNotStaged = ~0u;
+struct HexStageMap {
+    int slots = 0;                   // most elements of a node, at most kStageSlots
+    std::vector<uint32_t> src;       // [slots][num_nodes] first staged value (kNotStaged: none)
+    std::vector<int64_t> more_ptr;   // [num_nodes + 1] into more; empty when no node has more elements than slots
+    std::vector<uint32_t> more;
+};
+// order_pad: the element of each padded position (-1: none).
+HexStageMap hex_stage_map(int64_t num_nodes, const int32_t* conn, const std::vector<int>& order_pad);
 
 // Host set-up: element validity (positive volume, invertible J, Physics/Fem3DElementCube.cpp:169-211, 321-366),
 // lumped node masses (Physics/FemRepresentation.cpp:102-117), the node-pair block pattern and the

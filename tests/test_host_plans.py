@@ -1,4 +1,5 @@
-"""Runs the checks of the library's host side (tests/cpp/resident_plan_test.cpp, chip_share_test.cpp): no GPU."""
+"""Runs the checks of the library's host side (tests/cpp/resident_plan_test.cpp, hex_stage_test.cpp,
+chip_share_test.cpp): no GPU."""
 import os
 import subprocess
 import sys
@@ -16,6 +17,10 @@ def run(name):
 
 def test_resident_plans():
     run("resident_plan_test")
+
+
+def test_hex_staging_map():
+    run("hex_stage_test")
 
 
 def test_admission_of_solves():
