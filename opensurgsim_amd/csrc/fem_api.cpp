@@ -2576,23 +2576,35 @@ bool resident_columns(fem_ctx* c, const double* b, int64_t ncols, double* out, c
     return true;
 }
 
+// Whether [b, b + len) and [out, out + len) share no value.
+bool apart(const double* b, const double* out, int64_t len) { return b + len <= out || out + len <= b; }
+
 // Whether compliance columns take the one-launch CG: b and out apart (a solve that gives up starts again from b).
 bool use_resident_columns(fem_ctx* c, const double* b, const double* out, int64_t ncols) {
-    const int64_t len = ncols * c->ndof;
-    return use_resident(c, false) && c->num_instances == 0 && max_iters(c) >= 1 && (b + len <= out || out + len <= b);
+    return use_resident(c, false) && c->num_instances == 0 && max_iters(c) >= 1 && apart(b, out, ncols * c->ndof);
+}
+
+bool lu_in_place(const fem_ctx* c, const double* b, int64_t ncols, const double* out) {
+    return b == out || apart(b, out, ncols * c->ndof);
 }
 
 // Compliance columns through the band LU (LinearSparseSolveAndInverseLU::solve): each column of b with its
-// boundary rows zeroed into tmp (tmp_cols columns of ndof at a time), solved into out, boundary rows of the
-// solutions zeroed (DeformableRepresentation::applyCompliance, Physics/DeformableRepresentation.cpp:175-190).
-void compliance_lu(fem_ctx* c, const double* b, int64_t ncols, double* out, double* tmp, int64_t tmp_cols) {
+// boundary rows zeroed, solved in place in out, boundary rows of the solutions zeroed
+// (DeformableRepresentation::applyCompliance, Physics/DeformableRepresentation.cpp:175-190). All columns go to the solve
+// together. Where b and out overlap without being the same, tmp_cols columns at a time are copied aside to tmp first.
+// total: columns of the request that these are a part of.
+void compliance_lu(fem_ctx* c, const double* b, int64_t ncols, double* out, double* tmp, int64_t tmp_cols, int64_t total) {
     const int64_t n = c->ndof;
-    for (int64_t j0 = 0; j0 < ncols; j0 += tmp_cols) {
-        const int cnt = (int)std::min<int64_t>(tmp_cols, ncols - j0);
+    const bool in_place = lu_in_place(c, b, ncols, out);
+    const int64_t some = in_place ? int64_t(1) << 20 : tmp_cols;
+    for (int64_t j0 = 0; j0 < ncols; j0 += some) {
+        const int cnt = (int)std::min<int64_t>(some, ncols - j0);
+        double* const x = out + (size_t)j0 * n;
+        double* const y = in_place ? x : tmp;
         for (int j = 0; j < cnt; ++j)
-            launch_masked_copy(n, b + (size_t)(j0 + j) * n, c->bcmask.p, tmp + (size_t)j * n, c->stream);
-        launch_band_solve(c->lu, cnt, tmp, n, out + (size_t)j0 * n, n, c->stream, -1, ncols);
-        launch_zero_masked_rows(n, cnt, c->bcmask.p, out + (size_t)j0 * n, c->stream);
+            launch_masked_copy(n, b + (size_t)(j0 + j) * n, c->bcmask.p, y + (size_t)j * n, c->stream);
+        launch_band_solve(c->lu, cnt, y, n, x, n, c->stream, -1, total);
+        launch_zero_masked_rows(n, cnt, c->bcmask.p, x, c->stream);
     }
 }
 
@@ -2600,14 +2612,14 @@ void compliance_lu(fem_ctx* c, const double* b, int64_t ncols, double* out, doub
 // own work buffers. In the FP32 + refinement mode a remainder of fewer than 5 columns goes column by column
 // through the step's FP32 solver instead: on the 40^3 block a fixed-point constraint's 3 columns take 2.04 ms
 // that way against 2.19 ms in one 4-column FP64 pass, while a full 8-column pass costs 0.35 ms per column.
-void compliance_tet(fem_ctx* c, const double* b, int64_t ncols, double* out) {
+void compliance_tet(fem_ctx* c, const double* b, int64_t ncols, double* out, int64_t total) {
     const size_t n = (size_t)c->ndof;
     if (c->opt.linear_solver == FEM_LINEAR_SOLVER_LU) {
         ensure_lu(c);
         const int64_t tc = std::max<int64_t>(1, std::min<int64_t>(ncols, 64));
         DevBuf<double> tmp;
-        tmp.alloc(n * (size_t)tc);
-        compliance_lu(c, b, ncols, out, tmp.p, tc);
+        if (!lu_in_place(c, b, ncols, out)) tmp.alloc(n * (size_t)tc);
+        compliance_lu(c, b, ncols, out, tmp.p, tc, total);
         return;
     }
     if (c->opt.precision == FEM_PRECISION_FP32_REFINED) {
@@ -2635,8 +2647,8 @@ void compliance_tet(fem_ctx* c, const double* b, int64_t ncols, double* out) {
     mcg_columns(c, b, ncols, out, w);
 }
 
-// C b for num_columns device columns (column-major) on the context stream.
-void compliance_device(fem_ctx* c, const double* b, int64_t num_columns, double* out) {
+// C b for num_columns device columns (column-major) on the context stream; total: columns of the caller's request.
+void compliance_device(fem_ctx* c, const double* b, int64_t num_columns, double* out, int64_t total) {
     ensure_bc(c);
     alloc_precision_buffers(c);
     const size_t n = (size_t)c->ndof;
@@ -2648,7 +2660,7 @@ void compliance_device(fem_ctx* c, const double* b, int64_t num_columns, double*
     std::memcpy(saved_hex, c->predicted_hex, sizeof saved_hex);
     std::memcpy(saved_batch, c->b_predicted, sizeof saved_batch);
     if (c->kind != FEM_ELEMENT_HEX && c->num_instances == 0) {
-        compliance_tet(c, b, num_columns, out);
+        compliance_tet(c, b, num_columns, out, total);
     } else {
         for (int64_t j = 0; j < num_columns; ++j) compliance_column(c, b + (size_t)j * n, out + (size_t)j * n);
     }
@@ -2668,15 +2680,19 @@ int fem_apply_compliance(fem_ctx* c, const double* b, int64_t num_columns, doubl
         if (!c->have_operator) return fail(c, FEM_ERR_ORDER, "no system matrix yet: the solver has not stepped");
         HIPCHECK(hipSetDevice(c->device));
         const size_t n = (size_t)c->ndof;
-        // stage through device memory, up to 64 columns at a time
-        const int64_t chunk = std::min<int64_t>(std::max<int64_t>(num_columns, 1), 64);
+        // stage through device memory, up to 64 columns at a time; a request beyond the direct solver's solve by columns in parts as
+        // large as fit 256 MiB, as its tiled solve takes 3.9 ms for 513 columns of 3,240 DOFs together and 2.5 for 64
+        int64_t chunk = 64;
+        if (c->opt.linear_solver == FEM_LINEAR_SOLVER_LU && num_columns > kColumnSolves)
+            chunk = std::max<int64_t>(chunk, (int64_t(256) << 20) / (int64_t)(n * sizeof(double)));
+        chunk = std::min(std::max<int64_t>(num_columns, 1), chunk);
         DevBuf<double> db, dx;
         db.alloc(n * chunk);
         dx.alloc(n * chunk);
         for (int64_t j0 = 0; j0 < num_columns; j0 += chunk) {
             const int64_t m = std::min(chunk, num_columns - j0);
             db.upload(b + (size_t)j0 * n, n * m, c->stream);
-            compliance_device(c, db.p, m, dx.p);
+            compliance_device(c, db.p, m, dx.p, num_columns);
             HIPCHECK(hipMemcpyAsync(out + (size_t)j0 * n, dx.p, n * m * sizeof(double), hipMemcpyDeviceToHost,
                                     c->stream));
             HIPCHECK(hipStreamSynchronize(c->stream));
@@ -2691,7 +2707,7 @@ int fem_apply_compliance_device(fem_ctx* c, const double* b, int64_t num_columns
         if (num_columns < 0 || (num_columns > 0 && (!b || !out))) throw InvalidArg("null or negative columns");
         if (!c->have_operator) return fail(c, FEM_ERR_ORDER, "no system matrix yet: the solver has not stepped");
         HIPCHECK(hipSetDevice(c->device));
-        compliance_device(c, b, num_columns, out);
+        compliance_device(c, b, num_columns, out, num_columns);
         return FEM_OK;
     });
 }
@@ -2717,7 +2733,7 @@ int fem_apply_compliance_device_noalloc(fem_ctx* c, const double* b, int64_t num
         if (c->opt.linear_solver == FEM_LINEAR_SOLVER_LU) {
             ensure_lu(c, false);  // refactoring reuses the band storage of the last step's factorization
             const int64_t tc = (int64_t)(kNoAllocScratchBytes / ((size_t)c->ndof * sizeof(double)));
-            compliance_lu(c, b, num_columns, out, (double*)base, tc);
+            compliance_lu(c, b, num_columns, out, (double*)base, tc, num_columns);
             return FEM_OK;
         }
         const size_t work = column_work_doubles((size_t)c->ndof, c->res[0].columns) * sizeof(double);
@@ -2861,7 +2877,7 @@ int fem_constraint_compliance(fem_ctx* c, int64_t element, const double* coordin
                                     c->stream));
             launch_scatter_values(m * cnt, c->con_idx.p, c->con_val.p, c->con_b.p, c->stream);
         }
-        compliance_device(c, c->con_b.p, m, c->con_x.p);  // C H^T, boundary rows zero
+        compliance_device(c, c->con_b.p, m, c->con_x.p, m);  // C H^T, boundary rows zero
         std::vector<double> g((size_t)m * cnt);
         if (hcht && cnt > 0) {
             launch_gather_values(m * cnt, c->con_idx.p, c->con_x.p, c->con_out.p, c->stream);

@@ -713,9 +713,9 @@ void launch_band_solve(const DeviceBandLU& lu, int nrhs, const double* b, int64_
     // A workgroup per column: 1 column 0.32 ms against 1.43 with the tiled kernel at 3,240 DOFs, bandwidth 356; 64 columns
     // 0.52 against 2.53 (0.26 and 0.57 at 1,488 x 77, 0.88 and 4.9 at 5,184 x 470); 512 in one launch 1.9 against 4.1 (1.3 and
     // 2.3, 2.5 and 6.4). Two more rounds of 256 workgroups would bring the two level near 1,000. The line is drawn by the
-    // whole request (total), so that its results do not depend on how a caller cuts it. Columns of the identity stay with
-    // the tiled kernel, which skips the rows above them.
-    if (std::max<int64_t>(nrhs, total) <= 512 && identity_first < 0 && lu.bw <= kColumnMaxBw && lu.n <= kColumnMaxN) {
+    // whole request (total): every entry point passes it on, so that the results do not depend on how one cuts the request.
+    // Columns of the identity stay with the tiled kernel, which skips the rows above them.
+    if (std::max<int64_t>(nrhs, total) <= kColumnSolves && identity_first < 0 && lu.bw <= kColumnMaxBw && lu.n <= kColumnMaxN) {
         if (lu.bw <= 128) return solve_columns<2>(lu, nrhs, b, ldb, x, ldx, s);
         if (lu.bw <= 256) return solve_columns<4>(lu, nrhs, b, ldb, x, ldx, s);
         if (lu.bw <= 384) return solve_columns<6>(lu, nrhs, b, ldb, x, ldx, s);

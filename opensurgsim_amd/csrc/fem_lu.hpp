@@ -37,9 +37,10 @@ void launch_band_fill(DeviceBandLU& lu, int64_t num_blocks, const int* blk_row, 
 // In-place factorization of the band storage (the lower triangle is read): panels of 32 columns, each one launch of
 // LDS-tiled workgroups over the trailing bw x bw lower triangle; then L and the inverses of the diagonal blocks.
 void launch_band_factor(DeviceBandLU& lu, hipStream_t s);
+constexpr int64_t kColumnSolves = 512;
 // x = A^-1 b for nrhs columns (column j at b + j * ldb and x + j * ldx; x may alias b): forward substitution
-// with L and back substitution with U by 64-row blocks, one workgroup per column (up to 512 columns of a request, narrow
-// bands) or per 16 columns (4 below 64 columns). total: columns of the request that nrhs is a part of.
+// with L and back substitution with U by 64-row blocks, one workgroup per column (up to kColumnSolves columns of a request,
+// narrow bands) or per 16 columns (4 below 64 columns). total: columns of the request that nrhs is a part of.
 // identity_first >= 0: b holds columns identity_first .. of the identity, and the forward pass skips the rows
 // above each workgroup's first column (their solutions are zero).
 void launch_band_solve(const DeviceBandLU& lu, int nrhs, const double* b, int64_t ldb, double* x, int64_t ldx,

@@ -212,6 +212,45 @@ def test_lu_factor_and_solve_over_bandwidths(n):
     g.close()
 
 
+# bandwidths 134 and 1,022: a solve by columns up to 512 of a request, and the tiled solve at any number
+@pytest.mark.parametrize("n", [(7, 9, 3), (1, 15, 19)])
+def test_lu_columns_by_entry_point(n):
+    """The entry points for host and device columns and the one that allocates nothing solve a request the same way, however
+    they cut it: equal bit for bit. So do columns solved in place, and out that overlaps b."""
+    import torch
+    cfg = mg.config_linear_cpu(n)
+    g = make_gpu(cfg, scheme=femgpu.EULER_IMPLICIT, linear_solver=femgpu.LINEAR_SOLVER_LU)
+    assert g.step(1) == femgpu.FEM_OK
+    size = cfg.x0.size
+    B = np.random.default_rng(13).normal(size=(size, 700))
+    rows = torch.from_numpy(np.ascontiguousarray(B.T)).cuda()
+    for m in (1, 63, 64, 65, 512, 513, 700):
+        say("  %d DOF, %d columns" % (size, m))
+        host = g.apply_compliance(np.ascontiguousarray(B[:, :m])).reshape(size, m).T
+        got = []
+        for apply in (g.apply_compliance_device, g.apply_compliance_device_noalloc):
+            out = torch.zeros((m, size), dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            apply(rows.data_ptr(), m, out.data_ptr())
+            g.synchronize()
+            got.append(out.cpu().numpy())
+            same = rows[:m].clone()
+            torch.cuda.synchronize()
+            apply(same.data_ptr(), m, same.data_ptr())
+            g.synchronize()
+            got.append(same.cpu().numpy())
+        for x in got:
+            assert np.array_equal(x, host)
+    for apply in (g.apply_compliance_device, g.apply_compliance_device_noalloc):
+        both = torch.cat([torch.zeros_like(rows[:1]), rows[:5]])
+        torch.cuda.synchronize()
+        apply(both[1:].data_ptr(), 5, both.data_ptr())
+        g.synchronize()
+        want = g.apply_compliance(np.ascontiguousarray(B[:, :5])).reshape(size, 5).T
+        assert np.array_equal(both[:5].cpu().numpy(), want)
+    g.close()
+
+
 @pytest.mark.parametrize("n", [(119, 6, 6), (121, 6, 6), (122, 6, 6)])
 def test_lu_column_solve_at_its_largest(n):
     """17,640 and 17,934 DOFs, where a column fills the local memory, and 18,081, past the limit, against conjugate gradients
