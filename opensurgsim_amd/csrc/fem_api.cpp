@@ -516,21 +516,17 @@ void ensure_resident(fem_ctx* c, bool fp32) {
     if (plan.groups == 0) return;
     std::vector<unsigned char> h;
     std::vector<size_t> at;
-    auto add = [&](const auto& v) {
-        at.push_back(h.size());
-        const auto* p = reinterpret_cast<const unsigned char*>(v.data());
-        h.insert(h.end(), p, p + v.size() * sizeof(v[0]));
-        h.resize((h.size() + 255) & ~size_t(255));
+    auto add = [&](const auto&... v) {
+        h.reserve(((v.size() * sizeof(v[0]) + 255) + ...));
+        auto one = [&](const auto& w) {
+            at.push_back(h.size());
+            const auto* p = reinterpret_cast<const unsigned char*>(w.data());
+            h.insert(h.end(), p, p + w.size() * sizeof(w[0]));
+            h.resize((h.size() + 255) & ~size_t(255));
+        };
+        (one(v), ...);
     };
-    add(plan.group);
-    add(plan.row_node);
-    add(plan.halo_node);
-    add(plan.halo_pos);
-    add(plan.lane_k0);
-    add(plan.lane_info);
-    add(plan.row_lane);
-    add(plan.cols);
-    add(plan.wg);
+    add(plan.group, plan.row_node, plan.halo_node, plan.halo_pos, plan.lane_k0, plan.lane_info, plan.row_lane, plan.cols, plan.wg);
     r.mem.alloc(h.size());
     r.mem.upload(h.data(), h.size(), c->stream);
     // columns of a compliance solve (FP64) go side by side while CUs are left

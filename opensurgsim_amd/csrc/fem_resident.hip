@@ -623,6 +623,15 @@ int host_threads(int64_t n) {
     return (int)std::max<int64_t>(1, std::min<int64_t>({8, (int64_t)std::thread::hardware_concurrency(), n / 4096}));
 }
 
+// work() on that many threads, this one among them.
+template <typename Work>
+void on_threads(int threads, const Work& work) {
+    std::vector<std::future<void>> others;
+    for (int i = 1; i < threads; ++i) others.push_back(std::async(std::launch::async, work));
+    work();
+    for (auto& o : others) o.get();
+}
+
 // Splits order[i0, i1) into `parts` compact sets by recursive bisection along the longest extent; ends[p] is the end of set
 // p. Halves of large sets go to threads of their own.
 void bisect(int32_t* order, const double* x0, int64_t i0, int64_t i1, int parts, int64_t* ends, int threads) {
@@ -715,12 +724,11 @@ bool plan_group(ResidentPlan& plan, int g, int64_t i0, int64_t i1, int64_t n0, c
     return fits;
 }
 
-// The plan of nodes [n0, n0 + N) for nb blocks per lane and the given number of workgroups; empty when a workgroup would
-// overflow.
+// The plan of nodes [n0, n0 + N) for nb blocks per lane and the given number of workgroups, made by `threads` host threads; empty
+// when a workgroup would overflow.
 ResidentPlan try_plan(int64_t n0, int64_t N, const int32_t* rp, const int32_t* ci, const double* x0, bool fp32, int nb,
-                      int groups) {
+                      int groups, int threads) {
     ResidentPlan plan;
-    const int threads = host_threads(N);
     std::vector<int64_t> ends(groups + 1, 0);  // set g: [ends[g], ends[g + 1])
     plan.row_node.resize(N);
     std::iota(plan.row_node.begin(), plan.row_node.end(), (int32_t)n0);
@@ -740,12 +748,7 @@ ResidentPlan try_plan(int64_t n0, int64_t N, const int32_t* rp, const int32_t* c
             if (!plan_group(plan, g, ends[g], ends[g + 1], n0, rp, ci, local, halo[g])) fits = false;
         }
     };
-    {
-        std::vector<std::future<void>> others;
-        for (int i = 1; i < threads; ++i) others.push_back(std::async(std::launch::async, work));
-        work();
-        for (auto& o : others) o.get();
-    }
+    on_threads(threads, work);
     if (!fits) return {};
     std::vector<int32_t> pos(N);  // rows of the partition, counted from n0 as the nodes are
     for (int64_t i = 0; i < N; ++i) pos[plan.row_node[i] - n0] = (int32_t)(n0 + i);
@@ -773,11 +776,11 @@ constexpr int kResFill = kResThreads * 9 / 10;  // lanes asked of a workgroup: t
 
 // The plan of nodes [n0, n1) with nb blocks per lane on as few workgroups as take it, at most `most`.
 ResidentPlan fit_plan(int64_t n0, int64_t n1, const int32_t* rp, const int32_t* ci, const double* x0, bool fp32, int nb,
-                      int most) {
+                      int most, int threads) {
     const int64_t lanes = lanes_of(n0, n1, rp, nb);
     if (lanes > (int64_t)most * kResThreads) return {};
     for (int64_t groups = (lanes + kResFill - 1) / kResFill;; groups += std::max<int64_t>(1, groups / 16)) {
-        ResidentPlan p = try_plan(n0, n1 - n0, rp, ci, x0, fp32, nb, (int)std::min<int64_t>(groups, most));
+        ResidentPlan p = try_plan(n0, n1 - n0, rp, ci, x0, fp32, nb, (int)std::min<int64_t>(groups, most), threads);
         if (p.groups || groups >= most) return p;
     }
 }
@@ -788,7 +791,7 @@ ResidentPlan plan_resident(int64_t N, const int32_t* rp, const int32_t* ci, cons
     const int most = std::min(num_cus, kResMaxGroups);
     if (N <= 0 || N > (int64_t)most * kResThreads) return {};
     for (int nb : fp32 ? kNb32 : kNb64) {
-        ResidentPlan p = fit_plan(0, N, rp, ci, x0, fp32, nb, most);
+        ResidentPlan p = fit_plan(0, N, rp, ci, x0, fp32, nb, most, host_threads(N));
         if (p.groups) return p;
     }
     return {};
@@ -822,13 +825,22 @@ ResidentPlan plan_resident_batch(const std::vector<int64_t>& off, const int32_t*
     std::vector<std::array<int, 3>> inst;  // groups, first group, instance
     all.row_node.resize(off[M]);
     std::iota(all.row_node.begin(), all.row_node.end(), 0);
+    // an instance a thread, or a few large ones one after another by all threads (64 bodies of 25^3: 116 ms one after another by
+    // one thread)
+    const int threads = host_threads(off[M]);
+    std::vector<ResidentPlan> plans(M);
+    std::atomic<int> next{0};
+    on_threads(M < threads ? 1 : threads, [&] {
+        for (int m; (m = next++) < M;)
+            plans[m] = fit_plan(off[m], off[m + 1], rp, ci, x0, fp32, nb, most, M < threads ? threads : 1);
+    });
     for (int m = 0; m < M; ++m) {
-        ResidentPlan p = fit_plan(off[m], off[m + 1], rp, ci, x0, fp32, nb, most);
+        const ResidentPlan p = std::move(plans[m]);
         if (!p.groups) continue;
         all.instances[m] = 1;
         inst.push_back({p.groups, (int)all.group.size(), m});
         std::copy(p.row_node.begin(), p.row_node.end(), all.row_node.begin() + off[m]);
-        for (int4& g : p.group) {
+        for (int4 g : p.group) {
             g.z += (int)all.halo_node.size();
             all.group.push_back(g);
         }

@@ -116,10 +116,29 @@ void unused_nodes() {
             }
 }
 
+// Batches planned by several host threads: an instance a thread (24 of them), and all threads on each of a few.
+void batches_on_threads() {
+    for (int count : {24, 3})
+        for (bool fp32 : {false, true}) {
+            Mesh m;
+            std::vector<int64_t> off{0};
+            for (int i = 0; i < count; ++i) {
+                if (count == 3) m.grid(20, 19 + i, 21, 0);
+                else m.grid(9 + i % 5, 12, 11 + i % 3, 0);
+                off.push_back(m.nodes());
+            }
+            const ResidentPlan p = plan_resident_batch(off, m.rp.data(), m.ci.data(), m.x0.data(), fp32, 256);
+            check_plan("threads", m, p, m.nodes());
+            CHECK((int)p.wg.size() == p.groups && std::accumulate(p.launches.begin(), p.launches.end(), 0) == p.groups, "%d", count);
+            for (uint8_t planned : p.instances) CHECK(planned, "%d", count);
+        }
+}
+
 }  // namespace
 
 int main() {
     unused_nodes();
+    batches_on_threads();
     std::printf("%s: %d failed checks\n", failures ? "FAILED" : "ok", failures);
     return failures != 0;
 }
