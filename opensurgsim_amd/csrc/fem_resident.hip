@@ -800,6 +800,7 @@ ResidentPlan plan_resident(int64_t N, const int32_t* rp, const int32_t* ci, cons
 ResidentPlan plan_resident_batch(const std::vector<int64_t>& off, const int32_t* rp, const int32_t* ci, const double* x0,
                                  bool fp32, int num_cus) {
     const int most = std::min(num_cus, kResMaxGroups), M = (int)off.size() - 1;
+    if (off[M] > kResMaxRows) return {};
     // Fewest launches, each weighed by the time of an iteration with that many blocks per lane (3.8, 5.0, 6.2 us measured
     // in FP64, 3.8, 4.2, 5.2 us in FP32): the launches of a batch run one after another.
     const double weight[2][3] = {{3.8, 5.0, 6.2}, {3.8, 4.2, 5.2}};

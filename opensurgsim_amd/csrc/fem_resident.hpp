@@ -15,6 +15,7 @@ constexpr int kResMaxGroups = 256;    // workgroups of a solve (one per CU)
 constexpr int kResWords = 8;          // published words per workgroup and iteration (7 sums, 1 spare)
 constexpr int kResRing = 4;           // iterations whose published sums are kept apart
 constexpr int kResRowBytes64 = 48, kResRowBytes32 = 24;  // a node's w in the exchange, FP64 and FP32
+constexpr int64_t kResMaxRows = INT32_MAX / kResRowBytes64;  // nodes of a batch: the exchange is addressed by 32-bit offsets
 constexpr size_t kResSlotWords = (size_t)kResRing * kResMaxGroups * kResWords;
 
 // Partition of the block rows over the workgroups of a solve, with every lane's blocks and local columns.

@@ -134,11 +134,24 @@ void batches_on_threads() {
         }
 }
 
+// A batch of more nodes than the exchange addresses: one instance that would fit the chip beside unused nodes.
+void batch_beyond_the_exchange() {
+    for (int64_t nodes : {kResMaxRows, kResMaxRows + 1}) {
+        Mesh m;
+        m.grid(3, 3, 3, 0);
+        const std::vector<int64_t> off{0, m.nodes(), nodes};
+        m.rp.resize(nodes + 1, m.rp.back());
+        const ResidentPlan p = plan_resident_batch(off, m.rp.data(), m.ci.data(), m.x0.data(), false, 256);
+        CHECK((p.groups > 0) == (nodes == kResMaxRows), "%lld nodes", (long long)nodes);
+    }
+}
+
 }  // namespace
 
 int main() {
     unused_nodes();
     batches_on_threads();
+    batch_beyond_the_exchange();
     std::printf("%s: %d failed checks\n", failures ? "FAILED" : "ok", failures);
     return failures != 0;
 }
