@@ -279,7 +279,8 @@ def test_batch_gives_up_waiting(monkeypatch):
     assert np.linalg.norm(a[1] - b[1]) <= BOUND * np.linalg.norm(b[1])
 
 
-# fewer columns than fit side by side, more, and a mesh that takes the chip alone; a zero column among them
+# fewer columns than fit side by side, more, and a mesh that takes the chip alone; a zero column among them. With no wait allowed
+# the step gives up first where it has several workgroups, and the columns go on with the launch per iteration from the start
 @pytest.mark.parametrize("n, columns", [((3, 4, 3), 1), ((3, 4, 3), 70), ((12, 11, 13), 11), ((34, 33, 35), 3)])
 @pytest.mark.parametrize("wait", [None, "0"])
 def test_compliance_columns(monkeypatch, n, columns, wait):
@@ -301,3 +302,37 @@ def test_compliance_columns(monkeypatch, n, columns, wait):
         assert np.linalg.norm(got[0][:, j] - got[1][:, j]) <= BOUND * np.linalg.norm(got[1][:, j])
     for node in bc:
         assert not got[0][3 * node:3 * node + 3].any()
+
+
+@pytest.mark.parametrize("entry", ["device", "noalloc", "host"])
+def test_columns_give_up_waiting(monkeypatch, entry):
+    """Columns that give up themselves: the step before them is the direct solver's, so that they are the context's first
+    conjugate gradients. They are solved again by the multi-column CG, whose rounding is another one, and so equal those of a
+    context without one-launch solves bit for bit; with the usual limit the same calls do not."""
+    import torch
+    x0, tets, bc = block((12, 11, 13))
+    b = torch.from_numpy(np.random.RandomState(4).standard_normal((11, x0.size))).cuda()
+    got = {}
+    for kernels, wait in ((None, "0"), (None, None), ("fused", None)):
+        monkeypatch.setenv("FEM_CG_KERNELS", kernels) if kernels else monkeypatch.delenv("FEM_CG_KERNELS", raising=False)
+        monkeypatch.setenv("FEM_CG_WAIT_US", wait) if wait else monkeypatch.delenv("FEM_CG_WAIT_US", raising=False)
+        g = femgpu.FemGpu(0)
+        g.upload_mesh(femgpu.TET_COROTATIONAL, x0, tets, 5e4, 0.4, 1000.0)
+        g.add_bc_nodes(bc)
+        g.set_options(dt=1e-3, linear_solver=femgpu.LINEAR_SOLVER_LU)
+        assert g.step(1) == femgpu.FEM_OK
+        g.set_options(dt=1e-3, cg_tolerance=TOL)
+        if entry == "host":
+            got[kernels, wait] = g.apply_compliance(b.cpu().numpy().T).T
+        else:
+            out = torch.full_like(b, np.nan)
+            torch.cuda.synchronize()
+            (g.apply_compliance_device if entry == "device" else g.apply_compliance_device_noalloc)(
+                b.data_ptr(), len(b), out.data_ptr())
+            g.synchronize()
+            got[kernels, wait] = out.cpu().numpy()
+        g.close()
+    want = got["fused", None]
+    assert np.array_equal(got[None, "0"], want)
+    assert not np.array_equal(got[None, None], want)
+    assert np.linalg.norm(got[None, None] - want) <= BOUND * np.linalg.norm(want)
