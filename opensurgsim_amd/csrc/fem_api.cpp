@@ -2456,7 +2456,7 @@ void compliance_column(fem_ctx* c, const double* b, double* out) {
 // (device, column-major) are interleaved [dof][kw] with their boundary rows zeroed, solved together against
 // S64, and scattered back with the boundary rows of the solutions zeroed. In the FP32 + refinement mode a
 // remainder of fewer than 5 columns goes column by column through the step's FP32 solver instead: on the
-// 40^3 block a fixed-point constraint's 3 columns take 2.04 ms that way against 2.19 ms in one 4-column FP64
+// 40^3 block a fixed-point constraint's 3 columns take 0.88 ms that way and took 2.19 ms in one 4-column FP64
 // pass, while a full 8-column pass costs 0.35 ms per column.
 // Largest DOF count whose multi-column CG buffers fit the allocation-free workspace.
 int64_t noalloc_max_dof() {
@@ -2606,8 +2606,8 @@ void compliance_lu(fem_ctx* c, const double* b, int64_t ncols, double* out, doub
 
 // Compliance columns of a tetrahedral mesh through the multi-column FP64 CG (mcg_columns) on the context's
 // own work buffers. In the FP32 + refinement mode a remainder of fewer than 5 columns goes column by column
-// through the step's FP32 solver instead: on the 40^3 block a fixed-point constraint's 3 columns take 2.04 ms
-// that way against 2.19 ms in one 4-column FP64 pass, while a full 8-column pass costs 0.35 ms per column.
+// through the step's FP32 solver instead: on the 40^3 block a fixed-point constraint's 3 columns take 0.88 ms
+// that way and took 2.19 ms in one 4-column FP64 pass, while a full 8-column pass costs 0.35 ms per column.
 void compliance_tet(fem_ctx* c, const double* b, int64_t ncols, double* out, int64_t total) {
     const size_t n = (size_t)c->ndof;
     if (c->opt.linear_solver == FEM_LINEAR_SOLVER_LU) {

@@ -601,7 +601,7 @@ __global__ __launch_bounds__(256) void hex_cast_diag_kernel(int n, const double*
 }
 
 // q[row] += sum_k val[k] p[col[k]] over the localized external operator rows: one lane per row, every row listed
-// once, launched after the colour passes on the same stream.
+// once, launched after the gather on the same stream.
 template <typename TV>
 __global__ __launch_bounds__(256) void hex_ext_apply_kernel(int rows, const int* __restrict__ row,
                                                             const int* __restrict__ ptr, const int* __restrict__ col,

@@ -529,8 +529,8 @@ void launch_nb(const ResidentArgs& a, hipStream_t s, int wgs) {
 
 // Blocks per lane, smallest first: the smallest that fits the CUs is taken, as short lane loops over many CUs beat long
 // ones over few (whole steps, FP64 / FP32 + refinement: 21x18x20 cubes 181 us with 4 blocks against 213 with 7 and 222
-// with 10 / 191 with 7, 198 with 10, 225 with 20; 30^3 260, 269, 285 / 256, 265, 290). The largest are what 256
-// registers hold (180 of them blocks).
+// with 10 / 191 with 7, 198 with 10, 225 with 20; 30^3 260, 269, 285 / 256, 265, 290). The largest fill a lane's 256
+// registers, 180 of them with blocks; in FP64 with 10 the compiler spills 8 others (20 bytes a lane).
 constexpr int kNb64[] = {4, 7, 10};
 constexpr int kNb32[] = {7, 10, 20};
 

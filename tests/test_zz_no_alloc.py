@@ -3,7 +3,8 @@ fem_apply_compliance_device (Physics/DeformableRepresentation.cpp:175-190 is wha
 
 Two calls in a row on one GPU share its fixed workspace, the second on a smaller mesh with fewer columns,
 so stale contents of the first call must not leak into the second. In FP64 mode both entry points run the
-same multi-column CG kernels in the same batches, so the results are equal bit for bit; in the FP32 +
+same kernels (one-launch solves of the columns side by side at these sizes) in the same batches, so the results are
+equal bit for bit; in the FP32 +
 refinement mode the existing entry point sends a remainder of fewer than 5 columns through the FP32 step
 solver, and the two agree to the CG tolerance (bound 1e-9 relative at tolerance 1e-12).
 """
