@@ -1,7 +1,7 @@
 """ctypes wrapper of the FP64 CPU oracle (oracle/fem_oracle.cpp).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, by the smoke check and by the CPU-baseline leg
-of bench.py, always as the checker or the timed CPU baseline. The shipped library never
+of bench.py, always as what results are compared with or the timed CPU baseline. The shipped library never
 imports it.
 """
 import ctypes

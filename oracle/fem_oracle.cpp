@@ -3,7 +3,7 @@
 // TEST INFRASTRUCTURE ONLY. This file restates, in plain C++17 without Eigen, the reference
 // algorithm of the path (element kernels, sparsity pattern, assembly, boundary conditions,
 // Eigen-ConjugateGradient semantics, implicit Euler). It is linked only by tests/, by the
-// smoke check and by the CPU-baseline leg of bench.py, where it is the checker; it is never
+// smoke check and by the CPU-baseline leg of bench.py, which compares with it; it is never
 // part of the shipped library or of its compute path.
 //
 // Every function cites the reference file:line it follows (paths relative to the reference
